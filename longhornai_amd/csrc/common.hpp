@@ -30,6 +30,9 @@ typedef __attribute__((ext_vector_type(4))) int i32x4_t;
 typedef __attribute__((ext_vector_type(16))) int i32x16_t;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
+// Four floats at any 4-byte alignment (global 16-byte loads and stores need
+// no more): rows of any length and views at any element offset.
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_any_t;
 
 __device__ __forceinline__ f32x4_t mfma_bf16_16x16x32(u32x4_t a, u32x4_t b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
@@ -61,6 +64,59 @@ __device__ __forceinline__ f32x4_t mfma_fp8_16x16x32(u32x2_t a, u32x2_t b, f32x4
     return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(__builtin_bit_cast(long, a),
                                                       __builtin_bit_cast(long, b), c, 0, 0, 0);
 }
+
+// ---------------------------------------------------------------------------
+// Four adjacent elements of which the first cnt (1..4) exist.  FULL: all of
+// them, one access at any alignment; otherwise one by one, the missing ones
+// read as zero.  Callers branch on cnt == 4 once, around everything they do:
+// a branch per load makes the compiler wait for each before the next.
+// ---------------------------------------------------------------------------
+template <bool FULL>
+__device__ __forceinline__ f32x4_t load_f32x4(const float* p, int cnt) {
+    if constexpr (FULL) {
+        return *reinterpret_cast<const f32x4_any_t*>(p);
+    } else {
+        f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < cnt) v[j] = p[j];
+        return v;
+    }
+}
+template <bool FULL>
+__device__ __forceinline__ void store_f32x4(float* p, const f32x4_t& v, int cnt) {
+    if constexpr (FULL) {
+        *reinterpret_cast<f32x4_any_t*>(p) = v;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < cnt) p[j] = v[j];
+    }
+}
+template <bool FULL>
+__device__ __forceinline__ uint32_t load_u8x4(const uint8_t* p, int cnt) {
+    uint32_t w = 0;
+    if constexpr (FULL) {
+        __builtin_memcpy(&w, p, 4);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < cnt) w |= static_cast<uint32_t>(p[j]) << (8 * j);
+    }
+    return w;
+}
+template <bool FULL>
+__device__ __forceinline__ void store_u8x4(uint8_t* p, uint32_t w, int cnt) {
+    if constexpr (FULL) {
+        __builtin_memcpy(p, &w, 4);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < cnt) p[j] = static_cast<uint8_t>(w >> (8 * j));
+    }
+}
+struct Full { static constexpr bool value = true; };
+struct Part { static constexpr bool value = false; };
 
 // ---------------------------------------------------------------------------
 // Bit-exact conversions (same results as the reference software dtypes).
@@ -120,6 +176,22 @@ __device__ __forceinline__ uint8_t f32_to_e4m3(float value) {
     }
     if (e < -2) return static_cast<uint8_t>(s);
     return static_cast<uint8_t>(s | (rne_shift_u32(m | 0x800000u, 21 - e) & 0x7fu));
+}
+// The same rule on gfx950's v_cvt_pk_fp8_f32 for two values (bits 0..7 and
+// 8..15 of the result): the conversion rounds to nearest even with
+// denormals; saturation, the flush below 2^-9, NaN / inf and the sign are
+// made around it.  Equal to f32_to_e4m3 for every one of the 2^32 inputs
+// (checked on the device); about a third of its instructions.
+__device__ __forceinline__ uint32_t pack_e4m3x2(float a, float b) {
+    const float ma = fabsf(a), mb = fabsf(b);
+    const uint32_t w = static_cast<uint32_t>(
+        __builtin_amdgcn_cvt_pk_fp8_f32(fminf(ma, 448.0f), fminf(mb, 448.0f), 0, false));
+    auto edge = [](uint32_t c, float m, float v) {
+        c = m < 0x1p-9f ? 0u : c;
+        c = m < __builtin_inff() ? c : 0x7fu;
+        return c | ((__float_as_uint(v) >> 24) & 0x80u);
+    };
+    return edge(w & 0xffu, ma, a) | (edge((w >> 8) & 0xffu, mb, b) << 8);
 }
 // E4M3 -> fp32 (dtypes.hpp:160-196).
 __device__ __forceinline__ float e4m3_to_f32(uint8_t b) {

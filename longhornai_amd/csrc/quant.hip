@@ -13,6 +13,8 @@
 //   * no multiply-add is fused anywhere in this file.
 #include "common.hpp"
 
+#include <algorithm>
+
 #pragma clang fp contract(off)
 
 namespace lhq {
@@ -56,10 +58,27 @@ __device__ __forceinline__ uint8_t quant_mul(float x, float inv) {
     if constexpr (FP8) return f32_to_e4m3(x * inv);
     else return static_cast<uint8_t>(static_cast<int8_t>(sat_rint(x * inv, 127)));
 }
+// Four values with a reciprocal, as one word (value j in byte j).
 template <bool FP8>
-__device__ __forceinline__ uint8_t quant_div(float x, float s) {
-    if constexpr (FP8) return f32_to_e4m3(x / s);
-    else return static_cast<uint8_t>(static_cast<int8_t>(sat_rint(x / s, 127)));
+__device__ __forceinline__ uint32_t quant_mul4(float a, float b, float c, float d, float inv) {
+    if constexpr (FP8) {
+        return pack_e4m3x2(a * inv, b * inv) | (pack_e4m3x2(c * inv, d * inv) << 16);
+    } else {
+        auto q = [inv](float x) { return static_cast<uint32_t>(sat_rint(x * inv, 127)) & 0xffu; };
+        return q(a) | (q(b) << 8) | (q(c) << 16) | (q(d) << 24);
+    }
+}
+
+// rint(x / s) of a finite quotient below 256 in magnitude without the IEEE
+// division (about ten instructions an element): r = x * rs with rs = rcp(s)
+// (1 ulp) is within 256 * 2^-22 of x / s, and the correctly rounded quotient
+// within 256 * 2^-24 of it, so where r lies more than 2^-13 from a
+// half-integer both round to the same integer.  False (about 1 value in 4000,
+// and every NaN, infinite or larger quotient): the caller divides.
+__device__ __forceinline__ bool rint_quotient(float x, float rs, float& t) {
+    const float r = x * rs;
+    t = __builtin_rintf(r);
+    return fabsf(r) < 256.0f && fabsf(fabsf(r - t) - 0.5f) > 0x1p-13f;
 }
 
 // One workgroup per row: max-abs, scale = m / QMAX (1 if m == 0),
@@ -80,14 +99,14 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_kernel(const T* __restri
 }
 
 // fp32 rows whose length is a multiple of 4: 16-byte loads and 4-byte
-// stores; rows of up to 4 * 4 * kBlock elements stay in registers between
+// stores; rows of up to 8 * 4 * kBlock elements stay in registers between
 // the max-abs pass and the quantizing pass (one read of the row), longer
 // rows are read again (from L2).  Same rule as quant_per_row_kernel.
 template <bool FP8>
 __global__ __launch_bounds__(kBlock) void quant_per_row_f32_vec_kernel(const float* __restrict__ src,
                                                                        uint8_t* __restrict__ dst,
                                                                        float* __restrict__ scales, int dim) {
-    constexpr int R = 4;  // float4 chunks a thread keeps
+    constexpr int R = 8;  // float4 chunks a thread keeps
     const int64_t base = static_cast<int64_t>(blockIdx.x) * dim;
     const f32x4_t* s4 = reinterpret_cast<const f32x4_t*>(src + base);
     const int n4 = dim >> 2;
@@ -115,10 +134,7 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_f32_vec_kernel(const flo
     const float inv = 1.0f / scale;
     uint32_t* d4 = reinterpret_cast<uint32_t*>(dst + base);
     auto put = [&](int i, const f32x4_t& v) {
-        uint32_t w = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w |= static_cast<uint32_t>(quant_mul<FP8>(v[j], inv)) << (8 * j);
-        d4[i] = w;
+        d4[i] = quant_mul4<FP8>(v[0], v[1], v[2], v[3], inv);
     };
     if (cached) {
 #pragma unroll
@@ -132,152 +148,314 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_f32_vec_kernel(const flo
     if (threadIdx.x == 0) scales[blockIdx.x] = scale;
 }
 
-// bf16 rows whose length is a multiple of 8: 16-byte loads, the row is read
-// twice (the second pass hits in L2), 8-byte stores.
+// bf16 rows whose length is a multiple of 8: 16-byte loads, 8-byte stores;
+// rows of up to 4 * 8 * kBlock elements stay in registers between the two
+// passes, longer rows are read again (from L2).  Bound by memory: 2048 rows
+// of 4096 move 25 MB in 7.4 us at best (9.6 with a second read of the row).
 template <bool FP8>
 __global__ __launch_bounds__(kBlock) void quant_per_row_bf16_vec_kernel(const uint16_t* __restrict__ src,
                                                                         uint8_t* __restrict__ dst,
                                                                         float* __restrict__ scales,
                                                                         int dim) {
+    constexpr int R = 4;  // 16-byte chunks a thread keeps
     const int64_t base = static_cast<int64_t>(blockIdx.x) * dim;
     const u32x4_t* s4 = reinterpret_cast<const u32x4_t*>(src + base);
     const int n8 = dim >> 3;
+    const bool cached = n8 <= R * kBlock;
+    u32x4_t keep[R];
     float m = 0.0f;
-    for (int i = threadIdx.x; i < n8; i += kBlock) {
-        const u32x4_t v = s4[i];
+    auto scan = [&](const u32x4_t& v) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             m = amax(m, fabsf(__uint_as_float(v[j] << 16)));
             m = amax(m, fabsf(__uint_as_float(v[j] & 0xffff0000u)));
         }
+    };
+    if (cached) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int i = threadIdx.x + r * kBlock;
+            keep[r] = i < n8 ? s4[i] : u32x4_t{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) scan(keep[r]);
+    } else {
+        for (int i = threadIdx.x; i < n8; i += kBlock) scan(s4[i]);
     }
     m = block_max(m);
     const float qmax = FP8 ? 448.0f : 127.0f;
     const float scale = (m > 0.0f) ? m / qmax : 1.0f;
     const float inv = 1.0f / scale;
     u32x2_t* d2 = reinterpret_cast<u32x2_t*>(dst + base);
-    for (int i = threadIdx.x; i < n8; i += kBlock) {
-        const u32x4_t v = s4[i];
-        u32x2_t o;
+    auto put = [&](int i, const u32x4_t& v) {
+        auto lo = [](uint32_t w) { return __uint_as_float(w << 16); };
+        auto hi = [](uint32_t w) { return __uint_as_float(w & 0xffff0000u); };
+        d2[i] = u32x2_t{quant_mul4<FP8>(lo(v[0]), hi(v[0]), lo(v[1]), hi(v[1]), inv),
+                        quant_mul4<FP8>(lo(v[2]), hi(v[2]), lo(v[3]), hi(v[3]), inv)};
+    };
+    if (cached) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t lo = quant_mul<FP8>(__uint_as_float(v[j] << 16), inv);
-            const uint32_t hi = quant_mul<FP8>(__uint_as_float(v[j] & 0xffff0000u), inv);
-            const uint32_t pair = lo | (hi << 8);
-            if (j & 1) o[j >> 1] |= pair << 16;
-            else o[j >> 1] = pair;
+        for (int r = 0; r < R; ++r) {
+            const int i = threadIdx.x + r * kBlock;
+            if (i < n8) put(i, keep[r]);
         }
-        d2[i] = o;
+    } else {
+        for (int i = threadIdx.x; i < n8; i += kBlock) put(i, s4[i]);
     }
     if (threadIdx.x == 0) scales[blockIdx.x] = scale;
 }
 
 // Per-column scales (quant.cpp:75-96, 218-238), in three launches that need
-// no scratch memory: the scales array first holds the running max |x| of its
-// column as float bits (non-negative floats order like their bit patterns),
-// then the scale m / QMAX (1 where m == 0).
-//   (1) zero the scales;
-//   (2) a grid of (column block) x (row chunk) workgroups: each thread reduces
-//       VEC adjacent columns over kColRows rows with 16-byte loads, then one
-//       atomic max per column and chunk -- the max is order-independent and
-//       NaN never wins, so any split gives the reference's maximum;
-//   (3) turn each max into its scale.
-constexpr int kColRows = 64;
+// no scratch memory of their own:
+//   (1) a grid of (256 columns) x (row chunk) workgroups: each wave reduces
+//       a quarter of the chunk's rows, four adjacent columns per lane with
+//       16-byte loads, the waves meet in LDS, and the chunk's maxima go to
+//       dst, chunk i's at bytes [4 i cols, 4 (i + 1) cols) -- chunks are at
+//       least 64 rows, so they fit, and (3) overwrites them -- or, where one
+//       chunk holds all rows (dst may then be smaller), to the scales array.
+//       Maxima are order-independent and NaN never wins, so any split gives
+//       the reference's;
+//   (2) the maximum over the chunks, as the scale m / QMAX (1 where m == 0);
+//   (3) quantize: a thread takes its four columns' scales (and reciprocals)
+//       once and walks kQuantRows rows.
+// Bound by memory: the fp32 matrix is read twice (the second time partly
+// from the Infinity Cache) and the codes written.  K=4096, N=14336: 36 us
+// for (1) and 46 for (3); N=4097: 15 and 22.  (A thread per four columns of
+// a 64-row chunk with atomic maxima, and an IEEE division and a scale load
+// per element, took 111 us and 55 us in all.)
+// Any column count and 4-byte alignment; the last columns of a row whose
+// length is no multiple of four are taken one by one.
+constexpr int kQuantRows = 8;
 
-__global__ void zero_f32_kernel(float* __restrict__ p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0f;
-}
-
-template <int VEC>
-__global__ __launch_bounds__(kBlock) void col_max_kernel(const float* __restrict__ src,
-                                                         float* __restrict__ maxw, int rows, int cols) {
-    const int c0 = (blockIdx.x * kBlock + threadIdx.x) * VEC;
-    if (c0 >= cols) return;
-    float m[VEC];
+__global__ __launch_bounds__(kBlock) void col_max_kernel(const float* __restrict__ src, uint8_t* __restrict__ maxw,
+                                                         int rows, int cols, int chunk) {
+    __shared__ float part[4][256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c0 = blockIdx.x * 256 + lane * 4;
+    const int cnt = min(4, cols - c0);  // <= 0 past the last column
+    const int64_t chunks = (static_cast<int64_t>(rows) + chunk - 1) / chunk;
+    // (the grid's y extent is capped, so very tall inputs give a workgroup several chunks)
+    for (int64_t q = blockIdx.y; q < chunks; q += gridDim.y) {
+        float m[4] = {0.f, 0.f, 0.f, 0.f};
+        const int64_t r0 = q * chunk + wave * (chunk / 4);
+        const int64_t r1 = min<int64_t>(rows, r0 + chunk / 4);
+        // eight rows in flight; rows past the end read the last one again
+        auto scan = [&](auto full) {
+            for (int64_t r = r0; r < r1; r += 8) {
+                f32x4_t v[8];
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) m[j] = 0.0f;
-    // row chunks blockIdx.y, blockIdx.y + gridDim.y, ... (the grid's y extent
-    // is capped, so very tall inputs give a workgroup several chunks)
-    for (int r0 = blockIdx.y * kColRows; r0 < rows; r0 += gridDim.y * kColRows) {
-        const int r1 = min(rows, r0 + kColRows);
-        for (int r = r0; r < r1; ++r) {
-            const float* row = src + static_cast<int64_t>(r) * cols + c0;
-            if constexpr (VEC == 4) {
-                const f32x4_t v = *reinterpret_cast<const f32x4_t*>(row);
+                for (int i = 0; i < 8; ++i) v[i] = load_f32x4<full.value>(src + min(r + i, r1 - 1) * cols + c0, cnt);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) m[j] = amax(m[j], fabsf(v[j]));
-            } else {
-                m[0] = amax(m[0], fabsf(row[0]));
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) m[j] = amax(m[j], fabsf(v[i][j]));
             }
-        }
-    }
+        };
+        if (cnt >= 4) scan(Full{});
+        else if (cnt > 0) scan(Part{});
+        __syncthreads();
+        *reinterpret_cast<f32x4_t*>(&part[wave][lane * 4]) = f32x4_t{m[0], m[1], m[2], m[3]};
+        __syncthreads();
+        const int c = blockIdx.x * 256 + static_cast<int>(threadIdx.x);
+        float t = part[0][threadIdx.x];
 #pragma unroll
-    for (int j = 0; j < VEC; ++j)
-        if (m[j] > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(maxw + c0 + j), __float_as_uint(m[j]));
+        for (int w = 1; w < 4; ++w) t = amax(t, part[w][threadIdx.x]);
+        if (c < cols) __builtin_memcpy(maxw + 4 * (q * cols + c), &t, 4);
+    }
 }
 
+// A workgroup takes 64 columns, its waves every fourth chunk, four loads in
+// flight.  scales may be maxw itself (one chunk): a column's words are read
+// by its own workgroup, before it writes the scale.
 template <bool FP8>
-__global__ void col_finalize_kernel(float* __restrict__ scales, int cols) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= cols) return;
-    const float m = scales[c];
+__global__ __launch_bounds__(kBlock) void col_scale_kernel(const uint8_t* maxw, int chunks, float* scales, int cols) {
+    __shared__ float part[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = blockIdx.x * 64 + lane;
+    const int cc = min(c, cols - 1);
+    float m = 0.0f;
+    for (int q = wave; q < chunks; q += 16) {
+        float t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)  // past the last chunk: the last one again
+            __builtin_memcpy(&t[u], maxw + 4 * (static_cast<int64_t>(min(q + 4 * u, chunks - 1)) * cols + cc), 4);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) m = amax(m, t[u]);
+    }
+    part[wave][lane] = m;
+    __syncthreads();
+    if (wave != 0 || c >= cols) return;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) m = amax(m, part[w][lane]);
     const float qmax = FP8 ? 448.0f : 127.0f;
     scales[c] = (m > 0.0f) ? m / qmax : 1.0f;
 }
 
-// q = round(x / scale[c]); VEC adjacent elements per thread (VEC divides cols).
-template <bool FP8, int VEC>
-__global__ void quant_per_col_kernel(const float* __restrict__ src, const float* __restrict__ scales,
-                                     uint8_t* __restrict__ dst, int cols, int64_t n) {
-    const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * VEC;
-    if (i >= n) return;
-    const int c = static_cast<int>(i % cols);
-    if constexpr (VEC == 4) {
-        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(src + i);
-        const f32x4_t sc = *reinterpret_cast<const f32x4_t*>(scales + c);
-        uint32_t o = 0;
+// q = round(x / scale[c]).
+template <bool FP8>
+__global__ __launch_bounds__(kBlock) void quant_per_col_kernel(const float* __restrict__ src,
+                                                               const float* __restrict__ scales,
+                                                               uint8_t* __restrict__ dst, int rows, int cols) {
+    const int c0 = (blockIdx.x * kBlock + threadIdx.x) * 4;
+    if (c0 >= cols) return;
+    const int cnt = min(4, cols - c0);
+    auto body = [&](auto full) {
+        const f32x4_t sc = load_f32x4<full.value>(scales + c0, cnt);
+        f32x4_t rs;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o |= static_cast<uint32_t>(quant_div<FP8>(v[j], sc[j])) << (8 * j);
-        *reinterpret_cast<uint32_t*>(dst + i) = o;
-    } else {
-        dst[i] = quant_div<FP8>(src[i], scales[c]);
+        for (int j = 0; j < 4; ++j) rs[j] = __builtin_amdgcn_rcpf(sc[j]);
+        for (int64_t r0 = static_cast<int64_t>(blockIdx.y) * kQuantRows; r0 < rows;
+             r0 += static_cast<int64_t>(gridDim.y) * kQuantRows) {
+            const int64_t left = rows - r0;
+            f32x4_t v[kQuantRows];
+#pragma unroll
+            for (int i = 0; i < kQuantRows; ++i)
+                v[i] = load_f32x4<full.value>(src + (r0 + min<int64_t>(i, left - 1)) * cols + c0, cnt);
+#pragma unroll
+            for (int i = 0; i < kQuantRows; ++i) {
+                if (i >= left) break;
+                uint32_t o = 0;
+                if constexpr (FP8) {
+                    o = pack_e4m3x2(v[i][0] / sc[0], v[i][1] / sc[1]) |
+                        (pack_e4m3x2(v[i][2] / sc[2], v[i][3] / sc[3]) << 16);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float t;
+                        if (!rint_quotient(v[i][j], rs[j], t)) t = __builtin_rintf(v[i][j] / sc[j]);
+                        o |= (static_cast<uint32_t>(sat_rint(t, 127)) & 0xffu) << (8 * j);
+                    }
+                }
+                store_u8x4<full.value>(dst + (r0 + i) * cols + c0, o, cnt);
+            }
+        }
+    };
+    if (cnt == 4) body(Full{});
+    else body(Part{});
+}
+
+// Per-tensor, up to kSmallTensor elements (the activations of a decode
+// batch): one launch.  Every workgroup takes the maximum over the whole
+// tensor (from L2) and quantizes its own kSmallSlice elements; the first one
+// writes the scale.  24 x 4096 values: 6.1 us, where four launches (clear,
+// atomic max, quantize, finalize) took 10.4 us of kernels and their gaps.
+// The repeated reads grow with the size: 7.2 us at 2^17 values, where the
+// three launches below take 2.6 + 1.6 + 3.4 and two gaps.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallSlice = 4 * kSmallThreads;
+constexpr int64_t kSmallTensor = int64_t{1} << 17;
+
+template <bool FP8>
+__device__ __forceinline__ float tensor_scale(float m) {
+    return (m > 0.0f) ? m / (FP8 ? 448.0f : 127.0f) : 1.0f;
+}
+
+template <bool FP8>
+__global__ __launch_bounds__(kSmallThreads) void quant_tensor_small_kernel(const float* __restrict__ src,
+                                                                           uint8_t* __restrict__ dst, int n,
+                                                                           float* __restrict__ scale_out) {
+    __shared__ float part[kSmallThreads / 64];
+    const int mine = static_cast<int>(blockIdx.x) * kSmallSlice + 4 * static_cast<int>(threadIdx.x);
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    if (mine + 4 <= n) x = load_f32x4<true>(src + mine, 4);
+    else if (mine < n) x = load_f32x4<false>(src + mine, n - mine);
+    float m = 0.0f;
+    auto scan = [&m](const f32x4_t& v) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = amax(m, fabsf(v[j]));
+    };
+    const int n4 = n & ~3;
+    int i = 4 * static_cast<int>(threadIdx.x);
+    for (; i + 7 * kSmallSlice < n4; i += 8 * kSmallSlice) {  // eight loads in flight
+        f32x4_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = load_f32x4<true>(src + i + u * kSmallSlice, 4);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) scan(v[u]);
+    }
+    for (; i < n4; i += kSmallSlice) scan(load_f32x4<true>(src + i, 4));
+    if (static_cast<int>(threadIdx.x) < n - n4) m = amax(m, fabsf(src[n4 + threadIdx.x]));
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = part[0];
+#pragma unroll
+    for (int w = 1; w < kSmallThreads / 64; ++w) m = amax(m, part[w]);
+    const float scale = tensor_scale<FP8>(m);
+    const uint32_t w = quant_mul4<FP8>(x[0], x[1], x[2], x[3], 1.0f / scale);
+    if (mine + 4 <= n) store_u8x4<true>(dst + mine, w, 4);
+    else if (mine < n) store_u8x4<false>(dst + mine, w, n - mine);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
+}
+
+// Per-tensor, larger: (1) up to kMaxParts workgroups each put the maximum of
+// their grid-stride share in a word of dst (which has n > 4 kMaxParts bytes
+// and is overwritten by (3); no shared atomic), (2) one workgroup turns them
+// into the scale, (3) quantize with the reciprocal.  Bound by memory, the
+// tensor read twice: 4096 x 14336 fp32 96 us a call (with an atomic maximum
+// per workgroup, single loads and a software e4m3 conversion 153 us for int8
+// and 182 for fp8), 2048 x 4096 17 us (49).
+constexpr int kMaxParts = 2048;
+
+__global__ __launch_bounds__(kBlock) void tensor_max_kernel(const float* __restrict__ src, int64_t n,
+                                                            uint8_t* __restrict__ parts) {
+    float m = 0.0f;
+    auto scan = [&m](const f32x4_t& v) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = amax(m, fabsf(v[j]));
+    };
+    const int64_t step = static_cast<int64_t>(gridDim.x) * kBlock * 4, n4 = n & ~int64_t{3};
+    int64_t i = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * 4;
+    for (; i + 3 * step < n4; i += 4 * step) {
+        f32x4_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = load_f32x4<true>(src + i + u * step, 4);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) scan(v[u]);
+    }
+    for (; i < n4; i += step) scan(load_f32x4<true>(src + i, 4));
+    if (blockIdx.x == 0 && threadIdx.x < n - n4) m = amax(m, fabsf(src[n4 + threadIdx.x]));
+    m = block_max(m);
+    if (threadIdx.x == 0) __builtin_memcpy(parts + 4 * static_cast<int64_t>(blockIdx.x), &m, 4);
+}
+
+template <bool FP8>
+__global__ __launch_bounds__(kBlock) void tensor_scale_kernel(const uint8_t* __restrict__ parts, int count,
+                                                              float* __restrict__ scale_out) {
+    float m = 0.0f;
+    for (int i = threadIdx.x; i < count; i += kBlock) {
+        float p;
+        __builtin_memcpy(&p, parts + 4 * static_cast<int64_t>(i), 4);
+        m = amax(m, p);
+    }
+    m = block_max(m);
+    if (threadIdx.x == 0) *scale_out = tensor_scale<FP8>(m);
+}
+
+template <bool FP8>
+__global__ __launch_bounds__(kBlock) void quant_tensor_kernel(const float* __restrict__ src,
+                                                              uint8_t* __restrict__ dst, int64_t n,
+                                                              const float* __restrict__ scale) {
+    const float inv = 1.0f / *scale;
+    const int64_t step = static_cast<int64_t>(gridDim.x) * kBlock * 4;
+    int64_t i = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * 4;
+    for (; i + 3 * step + 4 <= n; i += 4 * step) {
+        f32x4_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = load_f32x4<true>(src + i + u * step, 4);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            store_u8x4<true>(dst + i + u * step, quant_mul4<FP8>(v[u][0], v[u][1], v[u][2], v[u][3], inv), 4);
+    }
+    for (; i < n; i += step) {
+        const int cnt = static_cast<int>(min<int64_t>(4, n - i));
+        const f32x4_t v = load_f32x4<false>(src + i, cnt);
+        store_u8x4<false>(dst + i, quant_mul4<FP8>(v[0], v[1], v[2], v[3], inv), cnt);
     }
 }
 
-// Per-tensor: (1) clear the max word, (2) atomic max of |x| bits (non-negative
-// floats order like their bit patterns; NaN is skipped), (3) quantize with the
-// reciprocal, (4) turn the max into the scale.  The max lives in scale_out
-// until step 4, so no scratch memory is needed.
-__global__ void clear_word_kernel(float* w) { *w = 0.0f; }
-
-__global__ void tensor_max_kernel(const float* __restrict__ src, int64_t n, float* __restrict__ maxw) {
-    float m = 0.0f;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * kBlock)
-        m = amax(m, fabsf(src[i]));
-    m = block_max(m);
-    if (threadIdx.x == 0 && m > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(maxw), __float_as_uint(m));
-}
-
-template <bool FP8>
-__global__ void quant_tensor_kernel(const float* __restrict__ src, uint8_t* __restrict__ dst, int64_t n,
-                                    const float* __restrict__ maxw) {
-    const float m = *maxw;
-    const float qmax = FP8 ? 448.0f : 127.0f;
-    const float scale = (m > 0.0f) ? m / qmax : 1.0f;
-    const float inv = 1.0f / scale;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * kBlock)
-        dst[i] = quant_mul<FP8>(src[i], inv);
-}
-
-template <bool FP8>
-__global__ void finalize_tensor_scale_kernel(float* w) {
-    const float m = *w;
-    const float qmax = FP8 ? 448.0f : 127.0f;
-    *w = (m > 0.0f) ? m / qmax : 1.0f;
-}
+// n = 0: the scale of an empty tensor.
+__global__ void unit_scale_kernel(float* w) { *w = 1.0f; }
 
 // Dequantizers: dst = decode(src) * scale (quant.cpp:47-50, 65-73, 98-105,
 // 190-193, 208-216, 240-249); MODE 0 = per-tensor, 1 = per-row, 2 = per-col.
@@ -321,22 +499,23 @@ __global__ void q4_pack_kernel(const float* __restrict__ src, const float* __res
     packed[t] = static_cast<uint8_t>((q0 & 0xf) | ((q1 & 0xf) << 4));
 }
 
-__global__ void q4_dequant_kernel(const uint8_t* __restrict__ packed, const float* __restrict__ scales,
-                                  float* __restrict__ dst, int N, int G, int64_t total) {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= total) return;
-    const int n = static_cast<int>(t % N);
-    const int64_t k = t / N;
-    const uint8_t b = packed[(k >> 1) * N + n];
-    const int nib = (k & 1) ? (b >> 4) : (b & 0xf);
-    const int q = nib >= 8 ? nib - 16 : nib;  // sign extension, quant.hpp:73-74
-    dst[t] = static_cast<float>(q) * scales[(k / G) * N + n];
-}
-
 // Asymmetric int4 (no reference counterpart): per (group, column) the range
 // is widened to contain 0, s = fp16((hi - lo) / 15) (1 if the range is empty,
 // at least 2^-14), z = clamp(rint(-lo / s), 0, 15); codes
 // u = clamp(rint(w / s) + z, 0, 15) use the fp16-rounded s.
+__device__ __forceinline__ void q4a_params(float lo, float hi, uint16_t& sh_bits, float& sq, float& zf) {
+    float s = (hi - lo) / 15.0f;
+    if (!(s > 0.0f)) s = 1.0f;
+    _Float16 sh = static_cast<_Float16>(s);  // RNE, like dtypes.hpp:17-55 for normal values
+    sq = static_cast<float>(sh);
+    if (sq < 0x1p-14f) {
+        sh = static_cast<_Float16>(0x1p-14f);
+        sq = 0x1p-14f;
+    }
+    zf = fminf(fmaxf(__builtin_rintf(-lo / sq), 0.0f), 15.0f);
+    sh_bits = __builtin_bit_cast(uint16_t, sh);
+}
+
 __global__ void q4a_params_kernel(const float* __restrict__ src, uint16_t* __restrict__ scales,
                                   uint8_t* __restrict__ zeros, int N, int G, int64_t total) {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -349,17 +528,8 @@ __global__ void q4a_params_kernel(const float* __restrict__ src, uint16_t* __res
         if (w < lo) lo = w;
         if (w > hi) hi = w;
     }
-    float s = (hi - lo) / 15.0f;
-    if (!(s > 0.0f)) s = 1.0f;
-    _Float16 sh = static_cast<_Float16>(s);  // RNE, like dtypes.hpp:17-55 for normal values
-    float sq = static_cast<float>(sh);
-    if (sq < 0x1p-14f) {
-        sh = static_cast<_Float16>(0x1p-14f);
-        sq = 0x1p-14f;
-    }
-    float zf = __builtin_rintf(-lo / sq);
-    zf = fminf(fmaxf(zf, 0.0f), 15.0f);
-    scales[t] = __builtin_bit_cast(uint16_t, sh);
+    float sq, zf;
+    q4a_params(lo, hi, scales[t], sq, zf);
     zeros[t] = static_cast<uint8_t>(zf);
 }
 
@@ -383,26 +553,174 @@ __global__ void q4a_pack_kernel(const float* __restrict__ src, const uint16_t* _
     packed[t] = static_cast<uint8_t>(b);
 }
 
-__global__ void q4a_dequant_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales,
-                                   const uint8_t* __restrict__ zeros, float* __restrict__ dst, int N, int G,
-                                   int64_t total) {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= total) return;
-    const int n = static_cast<int>(t % N);
-    const int64_t k = t / N;
-    const uint8_t b = packed[(k >> 1) * N + n];
-    const int u = (k & 1) ? (b >> 4) : (b & 0xf);
-    const int64_t gi = (k / G) * N + n;
-    dst[t] = static_cast<float>(u - static_cast<int>(zeros[gi])) * f16_to_f32(scales[gi]);
+// Dequantize int4: a thread owns four adjacent columns and kDeqPairs packed
+// rows, reading a 32-bit word of codes and writing two 16-byte runs of fp32
+// per packed row.  Bound by the write: K=4096, N=14336, G=128 writes 235 MB
+// in 44 us (a thread per element with two 64-bit divisions took 117).
+constexpr int kDeqPairs = 4;
+
+template <bool ASYM>
+__global__ __launch_bounds__(kBlock) void q4_dequant_kernel(const uint8_t* __restrict__ packed,
+                                                            const void* __restrict__ scales,
+                                                            const uint8_t* __restrict__ zeros,
+                                                            float* __restrict__ dst, int K, int N, int G) {
+    const int c0 = (blockIdx.x * kBlock + threadIdx.x) * 4;
+    if (c0 >= N) return;
+    const int cnt = min(4, N - c0);
+    struct Params {
+        f32x4_t s;
+        uint32_t z;
+    };
+    auto body = [&](auto full) {
+        constexpr bool F = full.value;
+        auto params = [&](int g) {  // a group's scales and zero points
+            const int64_t gi = static_cast<int64_t>(g) * N + c0;
+            Params p = {{0.f, 0.f, 0.f, 0.f}, 0u};
+            if constexpr (ASYM) {
+                const uint16_t* sp = static_cast<const uint16_t*>(scales) + gi;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (F || j < cnt) p.s[j] = f16_to_f32(sp[j]);
+                p.z = load_u8x4<F>(zeros + gi, cnt);
+            } else {
+                p.s = load_f32x4<F>(static_cast<const float*>(scales) + gi, cnt);
+            }
+            return p;
+        };
+        auto put = [&](int64_t k, uint32_t nib, const Params& p) {  // codes in the low nibbles of nib's bytes
+            f32x4_t v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int u = static_cast<int>((nib >> (8 * j)) & 0xfu);
+                // sign extension, quant.hpp:73-74
+                const int q = ASYM ? u - static_cast<int>((p.z >> (8 * j)) & 0xffu) : (u ^ 8) - 8;
+                v[j] = static_cast<float>(q) * p.s[j];
+            }
+            store_f32x4<F>(dst + k * N + c0, v, cnt);
+        };
+        const int pairs = K / 2;
+        for (int64_t i0 = static_cast<int64_t>(blockIdx.y) * kDeqPairs; i0 < pairs;
+             i0 += static_cast<int64_t>(gridDim.y) * kDeqPairs) {
+            uint32_t w[kDeqPairs];
+            Params p[kDeqPairs];
+#pragma unroll
+            for (int u = 0; u < kDeqPairs; ++u) {
+                const int64_t i = i0 + u < pairs ? i0 + u : pairs - 1;
+                w[u] = load_u8x4<F>(packed + i * N + c0, cnt);
+                p[u] = params(static_cast<int>(2 * i) / G);
+            }
+#pragma unroll
+            for (int u = 0; u < kDeqPairs; ++u) {
+                if (i0 + u >= pairs) break;
+                const int k = static_cast<int>(2 * (i0 + u));
+                put(k, w[u], p[u]);
+                if (G % 2 != 0) p[u] = params((k + 1) / G);  // an odd group may end inside the pair
+                put(k + 1, w[u] >> 4, p[u]);
+            }
+        }
+    };
+    if (cnt == 4) body(Full{});
+    else body(Part{});
+}
+
+template <bool ASYM>
+void launch_q4_dequant(const uint8_t* packed, const void* scales, const uint8_t* zeros, float* dst, int K, int N,
+                       int G, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(ceil_div(N, 4), kBlock)),
+                    static_cast<unsigned>(min(ceil_div(K / 2, kDeqPairs), 65535)));
+    q4_dequant_kernel<ASYM><<<grid, kBlock, 0, s>>>(packed, scales, zeros, dst, K, N, G);
+}
+
+// Groups of 32, 64, 128 or 256 rows, scales and codes in one pass over the
+// weights: a workgroup owns 64 adjacent columns of one group, wave w its rows
+// [w * R, (w + 1) * R) (G = 4 R), held in R registers per thread from one
+// coalesced 256-byte load per row; the four waves' extrema meet in LDS, every
+// thread then has its column's scale and writes the codes of its row pairs.
+// Bound by the fp32 read: K=4096, N=14336, G=128 reads 235 MB and writes 30.
+// (Two passes with a thread per column and per code byte, as the kernels
+// below still do for other group sizes, took 165 us a call; this one 54, 4.9
+// TB/s.  G = 32 / 64 / 256: 171 / 169 / 208 us before, 47 / 51 / 56 now.)
+// Any N and any alignment: a lane reads and writes single elements.
+template <bool ASYM, int R>
+__global__ __launch_bounds__(256) void q4_group_kernel(const float* __restrict__ src, void* __restrict__ scales,
+                                                       uint8_t* __restrict__ zeros, uint8_t* __restrict__ packed,
+                                                       int N, int NG) {
+    __shared__ float ext[2][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n = blockIdx.x * 64 + lane;
+    const int nc = min(n, N - 1);  // lanes past the last column read it again and write nothing
+    for (int g = blockIdx.y; g < NG; g += gridDim.y) {
+        const int64_t row0 = (static_cast<int64_t>(g) * 4 + wave) * R;
+        const float* p = src + row0 * N + nc;
+        float w[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) w[r] = p[static_cast<int64_t>(r) * N];
+        // the same compare-and-select as a serial scan: NaN never wins
+        float lo = 0.0f, hi = 0.0f;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if constexpr (ASYM) {
+                if (w[r] < lo) lo = w[r];
+                if (w[r] > hi) hi = w[r];
+            } else {
+                hi = amax(hi, fabsf(w[r]));
+            }
+        }
+        if constexpr (ASYM) ext[0][wave][lane] = lo;
+        ext[1][wave][lane] = hi;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (ASYM) {
+                const float l = ext[0][i][lane];
+                if (l < lo) lo = l;
+            }
+            hi = amax(hi, ext[1][i][lane]);
+        }
+        __syncthreads();
+        const int64_t gi = static_cast<int64_t>(g) * N + n;
+        float s, z = 0.0f;
+        if constexpr (ASYM) {
+            uint16_t sh;
+            q4a_params(lo, hi, sh, s, z);
+            if (wave == 0 && n < N) {
+                static_cast<uint16_t*>(scales)[gi] = sh;
+                zeros[gi] = static_cast<uint8_t>(z);
+            }
+        } else {
+            s = (hi > 0.0f) ? hi / 7.0f : 1.0f;
+            if (wave == 0 && n < N) static_cast<float*>(scales)[gi] = s;
+        }
+        const float rs = __builtin_amdgcn_rcpf(s);
+        auto code = [&](float x) -> uint32_t {
+            float t;
+            if (!rint_quotient(x, rs, t)) t = __builtin_rintf(x / s);
+            if constexpr (ASYM) return static_cast<uint32_t>(fminf(fmaxf(t + z, 0.0f), 15.0f));
+            else return static_cast<uint32_t>(sat_rint(t, 7)) & 0xfu;
+        };
+        uint8_t* q = packed + (row0 >> 1) * N + n;
+        if (n < N) {
+#pragma unroll
+            for (int r = 0; r < R; r += 2)
+                q[static_cast<int64_t>(r >> 1) * N] = static_cast<uint8_t>(code(w[r]) | (code(w[r + 1]) << 4));
+        }
+    }
+}
+
+template <bool ASYM>
+bool launch_q4_group(const float* src, void* scales, uint8_t* zeros, uint8_t* packed, int K, int N, int G,
+                     hipStream_t s) {
+    const int NG = K / G;
+    const dim3 grid(static_cast<unsigned>(ceil_div(N, 64)), static_cast<unsigned>(min(NG, 65535)));
+    if (G == 32) q4_group_kernel<ASYM, 8><<<grid, 256, 0, s>>>(src, scales, zeros, packed, N, NG);
+    else if (G == 64) q4_group_kernel<ASYM, 16><<<grid, 256, 0, s>>>(src, scales, zeros, packed, N, NG);
+    else if (G == 128) q4_group_kernel<ASYM, 32><<<grid, 256, 0, s>>>(src, scales, zeros, packed, N, NG);
+    else if (G == 256) q4_group_kernel<ASYM, 64><<<grid, 256, 0, s>>>(src, scales, zeros, packed, N, NG);
+    else return false;
+    return true;
 }
 
 inline unsigned blocks_for(int64_t n, int bs = kBlock) { return static_cast<unsigned>(ceil_div64(n, bs)); }
-
-// Per-tensor grid: enough workgroups to cover the chip, grid-stride beyond.
-inline unsigned tensor_grid(int64_t n) {
-    const int64_t b = ceil_div64(n, kBlock);
-    return static_cast<unsigned>(b < 2048 ? (b > 0 ? b : 1) : 2048);
-}
 
 template <bool FP8>
 int quantize_per_tensor(const float* src, uint8_t* dst, float* scale_out, int64_t n, void* stream,
@@ -410,12 +728,18 @@ int quantize_per_tensor(const float* src, uint8_t* dst, float* scale_out, int64_
     LHQ_REQUIRE(src && dst && scale_out, "%s: null pointer", who);
     LHQ_REQUIRE(n >= 0, "%s: negative n", who);
     hipStream_t s = as_stream(stream);
-    clear_word_kernel<<<1, 1, 0, s>>>(scale_out);
-    if (n > 0) {
-        tensor_max_kernel<<<tensor_grid(n), kBlock, 0, s>>>(src, n, scale_out);
-        quant_tensor_kernel<FP8><<<tensor_grid(n), kBlock, 0, s>>>(src, dst, n, scale_out);
+    if (n == 0) {
+        unit_scale_kernel<<<1, 1, 0, s>>>(scale_out);
+    } else if (n <= kSmallTensor) {
+        quant_tensor_small_kernel<FP8><<<blocks_for(n, kSmallSlice), kSmallThreads, 0, s>>>(
+            src, dst, static_cast<int>(n), scale_out);
+    } else {
+        const unsigned parts = static_cast<unsigned>(std::min<int64_t>(ceil_div64(n, 16 * kBlock), kMaxParts));
+        tensor_max_kernel<<<parts, kBlock, 0, s>>>(src, n, dst);
+        tensor_scale_kernel<FP8><<<1, kBlock, 0, s>>>(dst, static_cast<int>(parts), scale_out);
+        const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div64(n, 16 * kBlock), 1 << 20));
+        quant_tensor_kernel<FP8><<<grid, kBlock, 0, s>>>(src, dst, n, scale_out);
     }
-    finalize_tensor_scale_kernel<FP8><<<1, 1, 0, s>>>(scale_out);
     return check_launch(who);
 }
 
@@ -461,23 +785,19 @@ int quantize_per_col(const float* src, uint8_t* dst, float* scales, int rows, in
     LHQ_REQUIRE(rows >= 0 && cols >= 0, "%s: negative dims", who);
     if (cols == 0) return LHQ_OK;
     hipStream_t s = as_stream(stream);
-    // 16-byte loads need 4 | cols and aligned rows; scales and dst are then
-    // read / written in 16- and 4-byte units at multiples of 4 elements.
-    const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0 &&
-                     (reinterpret_cast<uintptr_t>(scales) & 15) == 0 && (reinterpret_cast<uintptr_t>(dst) & 3) == 0;
-    zero_f32_kernel<<<blocks_for(cols), kBlock, 0, s>>>(scales, cols);
+    // long chunks (little to merge) where they still make four workgroups per CU
+    const int64_t strips = ceil_div(cols, 256);
+    const int chunk = strips * ceil_div(rows, 256) >= 1024 ? 256 : strips * ceil_div(rows, 128) >= 1024 ? 128 : 64;
+    const int chunks = ceil_div(rows, chunk);
+    uint8_t* const maxw = chunks > 1 ? dst : reinterpret_cast<uint8_t*>(scales);
+    if (rows > 0)
+        col_max_kernel<<<dim3(static_cast<unsigned>(strips), static_cast<unsigned>(min(chunks, 65535))), kBlock, 0, s>>>(
+            src, maxw, rows, cols, chunk);
+    col_scale_kernel<FP8><<<blocks_for(cols, 64), kBlock, 0, s>>>(maxw, chunks, scales, cols);
     if (rows > 0) {
-        const int vcols = vec ? cols / 4 : cols;
-        const dim3 grid(static_cast<unsigned>(ceil_div(vcols, kBlock)),
-                        static_cast<unsigned>(min(ceil_div(rows, kColRows), 65535)));
-        if (vec) col_max_kernel<4><<<grid, kBlock, 0, s>>>(src, scales, rows, cols);
-        else col_max_kernel<1><<<grid, kBlock, 0, s>>>(src, scales, rows, cols);
-    }
-    col_finalize_kernel<FP8><<<blocks_for(cols), kBlock, 0, s>>>(scales, cols);
-    const int64_t n = static_cast<int64_t>(rows) * cols;
-    if (n > 0) {
-        if (vec) quant_per_col_kernel<FP8, 4><<<blocks_for(n / 4), kBlock, 0, s>>>(src, scales, dst, cols, n);
-        else quant_per_col_kernel<FP8, 1><<<blocks_for(n), kBlock, 0, s>>>(src, scales, dst, cols, n);
+        const dim3 grid(static_cast<unsigned>(ceil_div(ceil_div(cols, 4), kBlock)),
+                        static_cast<unsigned>(min(ceil_div(rows, kQuantRows), 65535)));
+        quant_per_col_kernel<FP8><<<grid, kBlock, 0, s>>>(src, scales, dst, rows, cols);
     }
     return check_launch(who);
 }
@@ -557,6 +877,7 @@ int lhq_q4_quantize_groupwise(const float* src, uint8_t* packed, float* scales, 
     LHQ_REQUIRE(q4_dims_ok(K, N, G), "q4_quantize_groupwise: need K,N,G > 0, K even, G | K (K=%d N=%d G=%d)",
                 K, N, G);
     hipStream_t s = as_stream(stream);
+    if (launch_q4_group<false>(src, scales, nullptr, packed, K, N, G, s)) return check_launch("q4_quantize_groupwise");
     const int64_t ns = static_cast<int64_t>(K / G) * N, np = static_cast<int64_t>(K / 2) * N;
     q4_scales_kernel<<<blocks_for(ns), kBlock, 0, s>>>(src, scales, N, G, ns);
     q4_pack_kernel<<<blocks_for(np), kBlock, 0, s>>>(src, scales, packed, N, G, np);
@@ -567,8 +888,7 @@ int lhq_q4_dequantize_groupwise(const uint8_t* packed, const float* scales, floa
                                 void* stream) {
     LHQ_REQUIRE(packed && scales && dst, "q4_dequantize_groupwise: null pointer");
     LHQ_REQUIRE(q4_dims_ok(K, N, G), "q4_dequantize_groupwise: bad dims (K=%d N=%d G=%d)", K, N, G);
-    const int64_t n = static_cast<int64_t>(K) * N;
-    q4_dequant_kernel<<<blocks_for(n), kBlock, 0, as_stream(stream)>>>(packed, scales, dst, N, G, n);
+    launch_q4_dequant<false>(packed, scales, nullptr, dst, K, N, G, as_stream(stream));
     return check_launch("q4_dequantize_groupwise");
 }
 
@@ -577,6 +897,7 @@ int lhq_q4a_quantize_groupwise(const float* src, uint8_t* packed, uint16_t* scal
     LHQ_REQUIRE(src && packed && scales && zeros, "q4a_quantize_groupwise: null pointer");
     LHQ_REQUIRE(q4_dims_ok(K, N, G), "q4a_quantize_groupwise: bad dims (K=%d N=%d G=%d)", K, N, G);
     hipStream_t s = as_stream(stream);
+    if (launch_q4_group<true>(src, scales, zeros, packed, K, N, G, s)) return check_launch("q4a_quantize_groupwise");
     const int64_t ns = static_cast<int64_t>(K / G) * N, np = static_cast<int64_t>(K / 2) * N;
     q4a_params_kernel<<<blocks_for(ns), kBlock, 0, s>>>(src, scales, zeros, N, G, ns);
     q4a_pack_kernel<<<blocks_for(np), kBlock, 0, s>>>(src, scales, zeros, packed, N, G, np);
@@ -587,8 +908,7 @@ int lhq_q4a_dequantize_groupwise(const uint8_t* packed, const uint16_t* scales, 
                                  float* dst, int K, int N, int G, void* stream) {
     LHQ_REQUIRE(packed && scales && zeros && dst, "q4a_dequantize_groupwise: null pointer");
     LHQ_REQUIRE(q4_dims_ok(K, N, G), "q4a_dequantize_groupwise: bad dims (K=%d N=%d G=%d)", K, N, G);
-    const int64_t n = static_cast<int64_t>(K) * N;
-    q4a_dequant_kernel<<<blocks_for(n), kBlock, 0, as_stream(stream)>>>(packed, scales, zeros, dst, N, G, n);
+    launch_q4_dequant<true>(packed, scales, zeros, dst, K, N, G, as_stream(stream));
     return check_launch("q4a_dequantize_groupwise");
 }
 

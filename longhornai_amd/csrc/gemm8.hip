@@ -20,9 +20,10 @@
 // XCD-aware: consecutive tiles of one group of tile rows land on one XCD so
 // its L2 sees the A rows and B columns they share.  Where the tiles fill at
 // most half the CUs, every workgroup takes a 256x128 half tile instead; up to
-// 32 rows gemm8_mid_kernel runs 16x16 MFMA blocks straight from global
-// memory with K split across its waves (the M = 1 GEMV of config 1 and
-// batched decode).
+// 64 rows gemm8_stream_kernel stages A in LDS and streams B past it (the
+// M = 1 GEMV and batched decode; where A's rows are not 16-byte aligned,
+// gemm8_mid_kernel reads both straight from global memory up to 32 rows).
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1086,6 +1087,54 @@ __global__ __launch_bounds__(NTHREADS) void gemm8_fp8_dma_kernel(Gemm8Args p) {
     dma_tile_fp8<STAGES>(p, ds_lds, tm * BM, tn * BN, acc);
 }
 
+// The epilogue of one 16x16 block at (r0, c0): D element j of lane l is row
+// r0 + 4 (l >> 4) + j, column c0 + (l & 15); rows past M and columns past N
+// are not stored.
+template <int EPI, int OP, typename Acc>
+__device__ __forceinline__ void store_block16(const Gemm8Args& p, const Acc& acc, int r0, int c0, int lane) {
+    const int c = c0 + (lane & 15);
+    if (c >= p.N) return;
+    if constexpr (OP == OP_FP8) {
+        float combined = p.alpha * p.As[0];  // gemm_quant.cpp:98
+        combined = combined * p.Bs[0];
+        float* Cp = static_cast<float*>(p.C);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = r0 + 4 * (lane >> 4) + j;
+            if (r >= p.M) continue;
+            const size_t o = static_cast<size_t>(r) * p.N + c;
+            // apply_beta (gemm_quant.cpp:12-21), then C += rescaled
+            const float base = (p.beta == 0.0f) ? 0.0f : (p.beta == 1.0f) ? Cp[o] : Cp[o] * p.beta;
+            Cp[o] = base + combined * acc[j];
+        }
+        return;
+    } else {
+        float bs = 0.0f;
+        if constexpr (EPI != EPI_I32) bs = p.Bs[c];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = r0 + 4 * (lane >> 4) + j;
+            if (r >= p.M) continue;
+            const size_t o = static_cast<size_t>(r) * p.N + c;
+            if constexpr (EPI == EPI_I32) {
+                static_cast<int32_t*>(p.C)[o] = acc[j];
+            } else {
+                float f = p.alpha * p.As[r];  // gemm_quant.cpp:44-46, left to right
+                f = f * bs;
+                f = f * static_cast<float>(acc[j]);
+                if constexpr (EPI == EPI_F32) {
+                    // apply_beta (gemm_quant.cpp:12-21), then C += rescaled
+                    float* Cp = static_cast<float*>(p.C);
+                    const float base = (p.beta == 0.0f) ? 0.0f : (p.beta == 1.0f) ? Cp[o] : Cp[o] * p.beta;
+                    Cp[o] = base + f;
+                } else {
+                    static_cast<uint16_t*>(p.C)[o] = f32_to_bf16(0.0f + f);
+                }
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Small- and mid-size int8 kernel (W8A8 with M <= kMidMaxM: the M = 1 GEMV
 // of config 1 and batched decode).  There the 256x256 tile kernel runs
@@ -1185,60 +1234,155 @@ __global__ __launch_bounds__(64 * W, MINW) void gemm8_mid_kernel(Gemm8Args p) {
 #pragma unroll
             for (int t = 0; t < T; ++t) acc[i][t] += red[w][i * T + t][lane];
 
-    // D element j of block (i, t) in lane l: row m0 + 16 i + 4 (l >> 4) + j,
-    // column n0 + 16 t + (l & 15)
-    if constexpr (OP == OP_FP8) {
-        float combined = p.alpha * p.As[0];  // gemm_quant.cpp:98
-        combined = combined * p.Bs[0];
-        float* Cp = static_cast<float*>(p.C);
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int c = n0 + 16 * t + (lane & 15);
-            if (c >= p.N) continue;
+    for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int i = 0; i < RB; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int r = m0 + 16 * i + 4 * (lane >> 4) + j;
-                    if (r >= p.M) continue;
-                    const size_t o = static_cast<size_t>(r) * p.N + c;
-                    // apply_beta (gemm_quant.cpp:12-21), then C += rescaled
-                    const float base = (p.beta == 0.0f) ? 0.0f : (p.beta == 1.0f) ? Cp[o] : Cp[o] * p.beta;
-                    Cp[o] = base + combined * acc[i][t][j];
-                }
+        for (int i = 0; i < RB; ++i) store_block16<EPI, OP>(p, acc[i][t], m0 + 16 * i, n0 + 16 * t, lane);
+}
+
+// ---------------------------------------------------------------------------
+// Up to 64 rows, A staged in LDS (gemm8_stream_kernel).  The kernel above reads
+// its A rows from L2 beside B, a 64-byte piece of 16 rows per load: at 16
+// rows that took 18.3 us where one row (every lane the same piece) took 13.4
+// (K = 4096, N = 14336, 58.7 MB of weights).  Here a workgroup of eight waves
+// (six for CT = 3) owns CT 16-column tiles, its waves are CT x KP (tile, K
+// part), and all of A's rows -- or, where they do not fit, a phase of KP * sp
+// k steps, the next one's in a second buffer -- go to LDS by DMA once, whole
+// 1 KiB runs of a row: 16-byte chunk c of row r in slot c ^ (r & 15), so the
+// 16 rows of an operand read meet no bank conflict.  Each wave keeps a
+// window of 16 B loads (16 KiB) in flight from its first k step to its last:
+// a step's registers are reloaded as soon as it is consumed.  Rows past M
+// are neither staged nor stored (their LDS words reach only their own D
+// rows).  The K parts' blocks meet in LDS in K order, the epilogue is the
+// kernel's above: int32 sums exactly, fp32 ones in a fixed order.
+// Measured (us a call, int8; before = the kernel above up to 32 rows, 256 x
+// 128 half tiles from 33): K = 4096, N = 14336 M = 1 14.3 -> 13.5, 16 18.8 ->
+// 14.7, 24 22.0 -> 15.6, 32 23.7 -> 16.0, 64 31.2 -> 19.8; K = N = 4096 M = 32
+// 13.6 -> 8.7, 64 28.6 -> 14.4; K = N = 8192 M = 1 15.8 -> 16.2, 16 19.8 ->
+// 18.9, 64 52.7 -> 25.1.  The weights' read bounds it (4.4 TB/s at M = 1).
+// ---------------------------------------------------------------------------
+constexpr int kStreamWindow = 16;
+constexpr int stream_waves(int CT) { return CT == 3 ? 6 : 8; }
+
+template <int EPI, int RB, int CT, int OP, int D>
+__global__ __launch_bounds__(64 * stream_waves(CT), 2) void gemm8_stream_kernel(Gemm8Args p, int sp, int phases,
+                                                                               int pitch) {
+    constexpr int W = stream_waves(CT), KP = W / CT;
+    using Acc = typename std::conditional<OP == OP_I8, i32x4_t, f32x4_t>::type;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t st_lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ct = wave % CT, kp = wave / CT;
+    const int r16 = lane & 15, kg = lane >> 4;
+    const int n0 = (static_cast<int>(blockIdx.x) * CT + ct) * 16;
+    const int steps = p.Kp / 64;
+    const int rows = min(16 * RB, p.M);
+    // (tiles past N read the last one's columns: B^T is padded to 256 rows,
+    // CT tiles from a multiple of CT may pass that)
+    const int last_col = p.tiles_n * BN - 1;
+    const uint8_t* const b_col = p.Bt + static_cast<size_t>(min(n0 + r16, last_col)) * p.Kp + 16 * kg;
+
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(p.A), 0, static_cast<int>(static_cast<uint32_t>(p.M) * static_cast<uint32_t>(p.K)),
+        0x00020000);
+    const int chunks = pitch / 16, buf_bytes = 16 * RB * pitch;
+    auto stage = [&](int phase) {
+        const int k0 = phase * KP * sp * 64;
+        uint8_t* const buf = st_lds + (phase & 1) * buf_bytes;
+        for (int r = wave; r < rows; r += W)
+            for (int c0 = 0; c0 < chunks; c0 += 64) {
+                const int slot = c0 + lane;
+                // k past K reads the row's last 16 bytes: B^T is zero there
+                const int k = min(k0 + 16 * (slot ^ (r & 15)), p.K - 16);
+                if (slot < chunks)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                        ra, (__attribute__((address_space(3))) void*)(buf + r * pitch + c0 * 16), 16,
+                        static_cast<uint32_t>(r) * static_cast<uint32_t>(p.K) + static_cast<uint32_t>(k), 0, 0, 0);
+            }
+    };
+    // the wave's k steps in order: j = 0 .. sp - 1 of phase 0, 1, ...
+    int pf_phase = 0, pf_j = 0;
+    auto next_b = [&]() {
+        const int s = min((pf_phase * KP + kp) * sp + pf_j, steps - 1);  // past the end: the last one, not used
+        if (++pf_j == sp) {
+            pf_j = 0;
+            ++pf_phase;
         }
-        return;
-    }
+        return *reinterpret_cast<const u32x4_t*>(b_col + static_cast<size_t>(s) * 64);
+    };
+    u32x4_t b[D];
+    stage(0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int c = n0 + 16 * t + (lane & 15);
-        if (c >= p.N) continue;
-        float bs = 0.0f;
-        if constexpr (EPI != EPI_I32) bs = p.Bs[c];
+    for (int u = 0; u < D; ++u) b[u] = next_b();
+    __builtin_amdgcn_sched_barrier(0);
+
+    Acc acc[RB];
 #pragma unroll
-        for (int i = 0; i < RB; ++i)
+    for (int i = 0; i < RB; ++i) acc[i] = Acc{};
+    // vmcnt(D): the D B loads issued after a phase's DMAs may still be in
+    // flight, the DMAs have landed; then every wave's have
+    static_assert(D == 16 || D == 8, "the wait below counts the window");
+    auto landed = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(D == 16 ? 0x4F70 : 0x0F78);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    const int groups = (sp + D - 1) / D;
+    for (int phase = 0; phase < phases; ++phase) {
+        // this phase's A is there, and every wave is done with the buffer
+        // that the next phase's goes to
+        landed();
+        if (phase + 1 < phases) stage(phase + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t* const abuf = st_lds + (phase & 1) * buf_bytes + r16 * pitch;
+        const int j_end = min(sp, steps - (phase * KP + kp) * sp);
+        auto group = [&](int g, auto reload) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int r = m0 + 16 * i + 4 * (lane >> 4) + j;
-                if (r >= p.M) continue;
-                const size_t o = static_cast<size_t>(r) * p.N + c;
-                if constexpr (EPI == EPI_I32) {
-                    static_cast<int32_t*>(p.C)[o] = acc[i][t][j];
-                } else {
-                    float f = p.alpha * p.As[r];  // gemm_quant.cpp:44-46, left to right
-                    f = f * bs;
-                    f = f * static_cast<float>(acc[i][t][j]);
-                    if constexpr (EPI == EPI_F32) {
-                        // apply_beta (gemm_quant.cpp:12-21), then C += rescaled
-                        float* Cp = static_cast<float*>(p.C);
-                        const float base = (p.beta == 0.0f) ? 0.0f : (p.beta == 1.0f) ? Cp[o] : Cp[o] * p.beta;
-                        Cp[o] = base + f;
-                    } else {
-                        static_cast<uint16_t*>(p.C)[o] = f32_to_bf16(0.0f + f);
+            for (int u = 0; u < D; ++u) {
+                const int j = g * D + u;
+                if (j < j_end) {  // uniform
+                    const int chunk = 4 * (kp * sp + j) + kg;
+                    u32x4_t a[RB];
+#pragma unroll
+                    for (int i = 0; i < RB; ++i)
+                        a[i] = *reinterpret_cast<const u32x4_t*>(abuf + 16 * i * pitch + 16 * (chunk ^ r16));
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) {
+                        if constexpr (OP == OP_I8) {
+                            acc[i] = mfma_i8_16x16x64(a[i], b[u], acc[i]);
+                        } else {
+                            // k 16 g .. + 7 of the step, then + 8 .. + 15, in
+                            // every lane group g (A and B alike)
+                            acc[i] = mfma_fp8_16x16x32(u32x2_t{a[i][0], a[i][1]}, u32x2_t{b[u][0], b[u][1]}, acc[i]);
+                            acc[i] = mfma_fp8_16x16x32(u32x2_t{a[i][2], a[i][3]}, u32x2_t{b[u][2], b[u][3]}, acc[i]);
+                        }
                     }
                 }
+                if constexpr (reload.value) b[u] = next_b();
             }
+        };
+        const bool last = phase + 1 == phases;
+        for (int g = 0; g < (last ? groups - 1 : groups); ++g) group(g, std::true_type{});
+        if (last) group(groups - 1, std::false_type{});
     }
+
+    Acc* const red = reinterpret_cast<Acc*>(st_lds);  // [kp - 1][ct][i][lane]
+    __syncthreads();
+    if (kp > 0) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i) red[(((kp - 1) * CT + ct) * RB + i) * 64 + lane] = acc[i];
+    }
+    __syncthreads();
+    if (kp != 0) return;
+#pragma unroll
+    for (int w = 0; w < KP - 1; ++w)
+#pragma unroll
+        for (int i = 0; i < RB; ++i) acc[i] += red[((w * CT + ct) * RB + i) * 64 + lane];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) store_block16<EPI, OP>(p, acc[i], 16 * i, n0, lane);
 }
 
 template <int EPI, int RB, int T, int W, int BATCH, int MINW, int OP = OP_I8>
@@ -1256,6 +1400,76 @@ int device_cus() {
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return 0;
     return cus;
+}
+
+// The stream kernel's shape for a call, or ct = 0 where it does not apply.
+constexpr size_t kStreamLds = 144 * 1024;  // A's buffers
+struct StreamPlan {
+    int ct = 0, sp = 0, phases = 0, pitch = 0;
+    size_t lds = 0;
+};
+StreamPlan plan_stream(const Gemm8Args& p, int rb) {
+    StreamPlan best;
+    static const int cus = std::max(device_cus(), 1);
+    static const int env_ct = env_int("LHQ_GEMM8_CT", 0);
+    const int steps = p.Kp / 64, nt = ceil_div(p.N, 16);
+    int64_t best_cost = 0;
+    for (int ct = 4; ct >= 1; --ct) {
+        if (env_ct && ct != env_ct) continue;
+        const int kp = stream_waves(ct) / ct;
+        StreamPlan t;
+        t.ct = ct;
+        t.sp = ceil_div(steps, kp);
+        t.phases = 1;
+        t.pitch = ceil_div(kp * t.sp * 64, 256) * 256;
+        if (static_cast<size_t>(16 * rb) * t.pitch > kStreamLds) {
+            // two buffers of whole windows
+            const int most = static_cast<int>(kStreamLds / 2 / (16 * rb)) / (64 * kp);
+            t.sp = most >= kStreamWindow ? most / kStreamWindow * kStreamWindow : most / 8 * 8;
+            if (t.sp < 8) continue;
+            t.phases = ceil_div(steps, kp * t.sp);
+            t.pitch = ceil_div(kp * t.sp * 64, 256) * 256;
+        }
+        const size_t a = static_cast<size_t>(t.phases > 1 ? 2 : 1) * 16 * rb * t.pitch;
+        t.lds = std::max(a, static_cast<size_t>(kp - 1) * ct * rb * 1024);
+        // rounds of the CUs times the tiles of a workgroup; ties to the wider
+        // one, which stages A less often
+        const int64_t wgs = ceil_div(nt, ct);
+        const int64_t cost = ceil_div64(wgs, static_cast<int64_t>(cus)) * ct;
+        if (best.ct == 0 || cost < best_cost) {
+            best = t;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+template <int EPI, int RB, int CT, int OP, int D>
+int launch_stream_d(const Gemm8Args& p, const StreamPlan& t, void* stream, const char* who) {
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm8_stream_kernel<EPI, RB, CT, OP, D>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (attr != hipSuccess)
+        return set_error(LHQ_ERR_HIP, "%s: dynamic LDS attribute: %s", who, hipGetErrorString(attr));
+    gemm8_stream_kernel<EPI, RB, CT, OP, D><<<ceil_div(ceil_div(p.N, 16), CT), 64 * stream_waves(CT), t.lds,
+                                              as_stream(stream)>>>(p, t.sp, t.phases, t.pitch);
+    return check_launch(who);
+}
+// a window of 8 where a wave has no more steps in a phase
+template <int EPI, int RB, int CT, int OP>
+int launch_stream_ct(const Gemm8Args& p, const StreamPlan& t, void* stream, const char* who) {
+    return t.sp <= 8 ? launch_stream_d<EPI, RB, CT, OP, 8>(p, t, stream, who)
+                     : launch_stream_d<EPI, RB, CT, OP, kStreamWindow>(p, t, stream, who);
+}
+
+template <int EPI, int RB, int OP>
+int launch_stream(const Gemm8Args& p, const StreamPlan& t, void* stream, const char* who) {
+    switch (t.ct) {
+        case 1: return launch_stream_ct<EPI, RB, 1, OP>(p, t, stream, who);
+        case 2: return launch_stream_ct<EPI, RB, 2, OP>(p, t, stream, who);
+        case 3: return launch_stream_ct<EPI, RB, 3, OP>(p, t, stream, who);
+        default: return launch_stream_ct<EPI, RB, 4, OP>(p, t, stream, who);
+    }
 }
 
 template <int EPI, int STAGES, bool M16>
@@ -1334,6 +1548,16 @@ int launch_gemm8(const uint8_t* A, const uint8_t* Bt, const float* As, const flo
     // of A before it reaches the MFMA
     static const int use_dma = env_int("LHQ_GEMM8_DMA", 1);
     static const int use_small = env_int("LHQ_GEMM8_SKINNY", 1);
+    // up to 64 rows: A staged in LDS, one pass over the weights (its loads
+    // need 16-byte aligned rows; from 65 rows a second pass costs what the
+    // half tiles do: K = N = 8192 M = 64 25 us, M = 65 on half tiles 53)
+    static const int env_stream = env_int("LHQ_GEMM8_STREAM", 64);
+    if (M <= env_stream && (OP == OP_I8 || K % BK == 0) && (reinterpret_cast<uintptr_t>(A) & 15) == 0) {
+        const StreamPlan t = plan_stream(p, M <= 16 ? 1 : M <= 32 ? 2 : 4);
+        if (t.ct && M <= 16) return launch_stream<EPI, 1, OP>(p, t, stream, who);
+        if (t.ct && M <= 32) return launch_stream<EPI, 2, OP>(p, t, stream, who);
+        if (t.ct) return launch_stream<EPI, 4, OP>(p, t, stream, who);
+    }
     if constexpr (OP == OP_FP8) {
         // up to 32 rows (K % 128 == 0): the mid-size kernel's 32 x 32 blocks.
         // K = 4096, N = 14336 (us, whole tiles / here): M = 1 40.9 / 15.9,

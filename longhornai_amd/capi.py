@@ -133,17 +133,19 @@ class _Lib:
                 "(the HIP backend has no fallback)")
         self.cdll = C.CDLL(path)
         self.path = path
+        self._fns = {}
         for name, args in SIGNATURES.items():
             fn = getattr(self.cdll, name)
             fn.argtypes = args
             fn.restype = _RESTYPES.get(name, _i)
+            self._fns[name] = fn
 
     def last_error(self) -> str:
         return self.cdll.lhq_last_error().decode()
 
     def call(self, name: str, *args) -> int:
         """Call an int-returning entry point and raise on a non-zero status."""
-        st = getattr(self.cdll, name)(*args)
+        st = self._fns[name](*args)
         if st != LHQ_OK:
             raise LhqError(name, st, self.last_error())
         return st

@@ -31,8 +31,16 @@ def lib():
     return capi.load()
 
 
+# The current stream's handle straight from the runtime binding:
+# torch.cuda.current_stream() builds a Stream object for it, 2.8 us of an 8 us
+# decode call against 0.3.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def dev(a: np.ndarray, device: str = "cuda") -> torch.Tensor:
@@ -71,16 +79,17 @@ def run(name: str, *args) -> None:
     until the call has enqueued its kernels; after that, torch's
     stream-ordered allocator cannot hand their memory to later work on the
     same stream before the kernels finish."""
-    keep = []
+    keep = []  # copies made here (the caller's tensors are held by args)
     conv = []
     for a in args:
-        if isinstance(a, np.ndarray):
-            a = dev(a)
         if isinstance(a, torch.Tensor):
-            keep.append(a)
             conv.append(a.data_ptr())
         elif a is None:
             conv.append(0)
+        elif isinstance(a, np.ndarray):
+            a = dev(a)
+            keep.append(a)
+            conv.append(a.data_ptr())
         else:
             conv.append(a)
     lib().call(name, *conv, stream())

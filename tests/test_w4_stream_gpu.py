@@ -1,0 +1,92 @@
+"""The W4A16 kernel for a few rows (weights streamed, rows staged in LDS) and
+the calls on both sides of its rule: 5 to 64 rows with ragged row blocks, one
+column tile to two rounds of the CUs, one K tile, K phases that end mid-window,
+G = 32 to 256, zero points, alpha / beta.
+
+Tolerance, against float64 on the same codes: the terms are x (144 + u - z) and
+-144 x, so a partial sum never exceeds 303 sum_k s |x|, and each of the at most
+2 K + 2 K/G + 8 additions (twice for fp32, hi and lo planes) rounds once
+(2^-24); plus half an ulp of the result: 2^-8 |want| in bf16, 2^-24 in fp32,
+whose hi + lo planes hold each activation to 2^-17.
+"""
+import numpy as np
+import pytest
+
+from tests import _data as D
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops(lib):
+    from longhornai_amd import ops as _ops
+    return _ops
+
+
+def _codes(K, N, G, seed):
+    g = D.rng(seed)
+    u = g.integers(0, 16, (K, N)).astype(np.uint8)
+    z = g.integers(0, 16, (K // G, N)).astype(np.uint8)
+    s = (0.01 * np.exp(0.3 * g.standard_normal((K // G, N)))).astype(np.float16)
+    return u, z, s, (u[0::2] | (u[1::2] << 4)).astype(np.uint8)
+
+
+def _products(x, u, z, s, G):
+    s64 = np.repeat(s.astype(np.float64), G, axis=0)
+    w = (u.astype(np.float64) - np.repeat(z.astype(np.float64), G, axis=0)) * s64
+    a = np.abs(x).astype(np.float64)
+    return x.astype(np.float64) @ w, 2.0 ** -24 * 303 * (a @ np.abs(s64)), a @ np.abs(w)
+
+
+@pytest.mark.parametrize("K,N,G", [
+    (128, 16, 32), (384, 33, 64), (2048, 5120, 32), (1152, 7000, 64), (1664, 13000, 32), (640, 28672, 64),
+    (2176, 3000, 128), (3072, 14336, 128), (3968, 6144, 128), (2048, 8192, 256), (1536, 28672, 256), (8192, 1000, 128),
+])
+@pytest.mark.parametrize("Ms", [(5, 8, 9, 13, 16, 17), (24, 32, 33, 48, 49, 64)])
+def test_bf16(oracle, ops, K, N, G, Ms):
+    u, z, s, packed = _codes(K, N, G, K + N)
+    w = ops.prepack_w4_asym(ops.dev(packed), ops.dev(s.view(np.uint16)), ops.dev(z), K, N, G)
+    xb = D.to_bf16_bits(oracle, D.normal((64, K), 1.0, K))
+    want, unit, _ = _products(D.bf16_bits_to_f32(xb), u, z, s, G)
+    for M in Ms:
+        C = ops.host(ops.gemm_w4a16_bf16(ops.dev(np.ascontiguousarray(xb[:M])), w), np.uint16)
+        got = D.bf16_bits_to_f32(C).astype(np.float64)
+        assert np.isfinite(got).all()
+        bound = (2 * K + 2 * K // G + 8) * unit[:M] + 2.0 ** -8 * np.abs(want[:M])
+        assert (np.abs(got - want[:M]) <= bound).all(), M
+        assert np.linalg.norm(got - want[:M]) <= 2.5e-3 * np.linalg.norm(want[:M]), M
+
+
+@pytest.mark.parametrize("K,N,G,alpha,beta", [
+    (128, 16, 128, 1.0, 0.0), (1152, 300, 128, 0.5, 2.0), (1024, 14336, 128, 1.0, 0.0), (2048, 8192, 256, 1.0, -1.0),
+    (8192, 1000, 128, 1.0, 0.0),
+])
+def test_f32(ops, K, N, G, alpha, beta):
+    u, _, s, packed = _codes(K, N, G, K + N)
+    s32 = s.astype(np.float32)
+    w = ops.prepack_w4_sym(ops.dev((packed ^ 0x88).astype(np.uint8)), ops.dev(s32), K, N, G)  # codes as signed nibbles
+    x = D.normal((32, K), 1.0, K)
+    C0 = D.normal((32, N), 1.0, 5)
+    prod, unit, mag = _products(x, u, np.full_like(u[: K // G], 8), s, G)
+    for M in (5, 8, 9, 16, 17, 32):
+        C = ops.dev(C0[:M])
+        ops.run("lhq_gemm_w4a16", ops.dev(x[:M]), w.qweight, w.scales, C, M, N, K, G, alpha, beta)
+        got = ops.host(C).astype(np.float64)
+        want = alpha * prod[:M] + beta * C0[:M]
+        bound = abs(alpha) * ((4 * K + 2 * K // G + 8) * unit[:M] + 2.0 ** -17 * mag[:M]) + 2.0 ** -22 * (
+            np.abs(want) + np.abs(beta * C0[:M]))
+        assert (np.abs(got - want) <= bound).all(), M
+        assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want), M
+
+
+def test_non_finite_rows_stay_apart(oracle, ops):
+    K, N, G, M = 1152, 7000, 64, 17
+    u, z, s, packed = _codes(K, N, G, 2)
+    w = ops.prepack_w4_asym(ops.dev(packed), ops.dev(s.view(np.uint16)), ops.dev(z), K, N, G)
+    x = D.normal((M, K), 1.0, 3)
+    x[4, 700], x[16, 1151] = np.inf, np.nan
+    got = D.bf16_bits_to_f32(ops.host(ops.gemm_w4a16_bf16(ops.dev(D.to_bf16_bits(oracle, x)), w), np.uint16))
+    bad = ~np.isfinite(got)
+    assert bad[16].all() and bad[4].any()
+    bad[[4, 16]] = False
+    assert not bad.any()

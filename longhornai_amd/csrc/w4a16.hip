@@ -2767,10 +2767,14 @@ int f32_thin_layout(const W4Args& a, int M) {
     return N >= 40000 ? 0 : N >= 16384 ? 2 : N >= 10240 ? 3 : 0;
 }
 
+// The tile kernel's shapes, and where it is the faster one for a plain or
+// batched call (a grouped one: grouped_uses_tiles).
+bool mma_takes(const W4Args& a, int64_t rows) {
+    return a.G >= kW4TileK && a.K % kW4TileK == 0 && rows * a.K < (int64_t{1} << 31);
+}
 bool mma_applies(const W4Args& a, int64_t rows, double rows_per_block) {
     static const int env = tuning_knob("LHQ_W4_MMA", -1);
-    if (env == 0) return false;
-    if (a.G < kW4TileK || a.K % kW4TileK != 0 || rows * a.K >= (int64_t{1} << 31)) return false;
+    if (env == 0 || !mma_takes(a, rows)) return false;
     // The 16-row kernel re-reads the activation rows for every column tile
     // (rows * K * 2 bytes per 16 columns, from L2), the tile kernel once per
     // 256 columns through LDS; the tile kernel has fewer workgroups.
@@ -3071,8 +3075,25 @@ W4Args grouped_args(const uint16_t* A, const int32_t* offsets, const uint8_t* co
     a.row_capacity = row_capacity;
     return a;
 }
+// Tiles for a grouped launch with a workspace.  The persistent launch shares its tiles out
+// over the CUs, so with a 256-column tile per CU or more among all groups'
+// columns (or long K behind fewer) it wins from about 12 rows per group on,
+// where every group still wastes most of its 64-row tile: the 16-row kernel
+// reads the rows from L2 for every column tile, and the weights again for
+// each 16 of them.  us of a MoE layer, that launch on the 16-row kernel / on
+// tiles, at 16 and 40 rows per group:
+//   64 experts, gate / up K=4096, 2 x 1792 columns: 299 / 267, 486 / 376;
+//               down K=1792, 4096 columns: 299 / 283, 486 / 434
+//   8 experts,  gate / up K=2048, 2 x 5632: 71 / 69, 114 / 86;
+//               down K=14336, 4096 (128 tiles): 274 / 269, 449 / 408
+//   but 8 experts of K=1024, 2 x 2048 (128 tiles) 37 / 41, 48 / 52, and
+//   down K=5632, 2048 (64 tiles) 71 / 77, 114 / 114
 bool grouped_uses_tiles(const W4Args& a) {
-    return mma_applies(a, a.row_capacity, static_cast<double>(a.row_capacity) / a.num_groups);
+    const double rows = static_cast<double>(a.row_capacity) / a.num_groups;
+    if (mma_applies(a, a.row_capacity, rows)) return true;
+    const int64_t tiles = static_cast<int64_t>(a.num_groups) * a.Nt / 16;
+    return mma_takes(a, a.row_capacity) && rows >= 16.0 &&
+           (tiles >= device_cus() || tiles * a.K >= (int64_t{3} << 19));
 }
 
 // Partial-sum slots a persistent grouped launch can use: a split of R = T
@@ -3099,9 +3120,11 @@ int grouped_w4(const char* who, const uint16_t* A, const int32_t* offsets, const
     // at most min(num_groups, row_capacity) groups hold rows, so
     // sum_e ceil(rows_e / B) <= ceil(row_capacity / B) + live_groups for row blocks of B
     const int live_groups = std::min(num_groups, row_capacity);
-    if (grouped_uses_tiles(a)) {
-        if (ws && ws_bytes >= kPkSlotBytes) {
-            LHQ_REQUIRE((reinterpret_cast<uintptr_t>(ws) & 15) == 0, "%s: workspace not 16-byte aligned", who);
+    const bool pk = ws && ws_bytes >= kPkSlotBytes, aligned = (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
+    if (mma_applies(a, row_capacity, static_cast<double>(row_capacity) / num_groups) ||
+        (pk && aligned && grouped_uses_tiles(a))) {
+        if (pk) {
+            LHQ_REQUIRE(aligned, "%s: workspace not 16-byte aligned", who);
             return launch_mma_pk<SWI>(a, ws, ws_bytes / kPkSlotBytes, as_stream(stream), who);
         }
         return launch_mma<true, SWI>(a, row_capacity, live_groups, 1, as_stream(stream), who);

@@ -3456,14 +3456,19 @@ int gemm_w4a16_f32(const char* who, const float* A, const uint8_t* qweight, cons
     LHQ_REQUIRE(ws || ws_cap <= 0, "%s: null workspace with %lld bytes", who, static_cast<long long>(ws_cap));
     if (M == 0) return LHQ_OK;
     W4Args a = make_args(A, qweight, scales, nullptr, C, M, N, K, G, alpha, beta);
-    if (const int rb = w4_stream_rb(a, true)) return launch_w4_stream(a, true, rb, as_stream(stream), who);
+    // a misaligned workspace goes by the plan first, which refuses it where it
+    // would split K, whichever kernel then takes the call
+    const int rb = w4_stream_rb(a, true);
+    const bool aligned = (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
+    if (rb && aligned) return launch_w4_stream(a, true, rb, as_stream(stream), who);
     if (ws_cap > 0) {
         const TilePlan t = plan_thin_f32(a, ws_cap);
         if (t.split) {
-            LHQ_REQUIRE((reinterpret_cast<uintptr_t>(ws) & 15) == 0, "%s: workspace not 16-byte aligned", who);
+            LHQ_REQUIRE(aligned, "%s: workspace not 16-byte aligned", who);
             return launch_split_f32(a, t, ws, as_stream(stream), who);
         }
     }
+    if (rb) return launch_w4_stream(a, true, rb, as_stream(stream), who);
     const int thin = f32_thin_layout(a, M);
     if (!thin && mma_applies(a, M, M)) return launch_mma_f32(a, as_stream(stream), who);
     if (thin == 2) return M <= 16 ? launch_mma_f32_rb<2, 1>(a, as_stream(stream), who)
@@ -3485,12 +3490,16 @@ int gemm_w4a16_bf16_plan(const char* who, const uint16_t* A, const uint8_t* qwei
     LHQ_REQUIRE(ws || ws_cap <= 0, "%s: null workspace with %lld bytes", who, static_cast<long long>(ws_cap));
     if (M == 0) return LHQ_OK;
     W4Args a = make_args(A, qweight, scales, zeros, C, M, N, K, G, 1.0f, 0.0f);
-    if (const int rb = w4_stream_rb(a, false)) return launch_w4_stream(a, false, rb, as_stream(stream), who);
+    // (a misaligned workspace: as in gemm_w4a16_f32)
+    const int rb = w4_stream_rb(a, false);
+    const bool aligned = (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
+    if (rb && aligned) return launch_w4_stream(a, false, rb, as_stream(stream), who);
     const TilePlan t = plan_thin(a, ws ? ws_cap : 0);
     if (t.split) {
-        LHQ_REQUIRE((reinterpret_cast<uintptr_t>(ws) & 15) == 0, "%s: workspace not 16-byte aligned", who);
+        LHQ_REQUIRE(aligned, "%s: workspace not 16-byte aligned", who);
         return launch_split(a, t, ws, as_stream(stream), who);
     }
+    if (rb) return launch_w4_stream(a, false, rb, as_stream(stream), who);
     if (mma_applies(a, M, M)) return launch_mma<false>(a, M, 0, 1, as_stream(stream), who);
     return launch_w4<false, true, false>(a, 1, as_stream(stream));
 }

@@ -90,3 +90,28 @@ def test_non_finite_rows_stay_apart(oracle, ops):
     assert bad[16].all() and bad[4].any()
     bad[[4, 16]] = False
     assert not bad.any()
+
+
+@pytest.mark.parametrize("M,K,N", [(16, 8192, 8192), (8, 8192, 4096), (16, 4096, 8192)])
+def test_misaligned_workspace_is_refused_as_before(ops, M, K, N):
+    """Where the tiles would split K over it, a workspace that is not 16-byte
+    aligned is an error, also where this kernel takes the call."""
+    from longhornai_amd import capi
+    G, L = 128, ops.lib()
+    qw = ops.dev(np.zeros(K * ((N + 15) // 16 * 16) // 2, np.uint8))
+    sc = ops.dev(np.zeros((K // G) * ((N + 15) // 16 * 16), np.float32))
+    zs = ops.dev(np.zeros((K // G) * ((N + 15) // 16 * 16), np.uint8))
+    A, C = ops.dev(np.zeros((M, K), np.float32)), ops.dev(np.zeros((M, N), np.float32))
+    refused = 0
+    for name, need, rest in [
+        ("lhq_gemm_w4a16_bf16_ws", L.lhq_gemm_w4a16_bf16_workspace_bytes(M, N, K, G), ()),
+        ("lhq_gemm_w4a16_ws", L.lhq_gemm_w4a16_workspace_bytes(M, N, K, G), (1.0, 0.0)),
+    ]:
+        if need <= 0:
+            continue
+        ws = ops.dev(np.zeros(need + 16, np.uint8))
+        weights = (qw, sc, zs) if "bf16" in name else (qw, sc)
+        with pytest.raises(capi.LhqError, match="16-byte aligned"):
+            ops.run(name, A, *weights, C, M, N, K, G, *rest, ws[4:], need)
+        refused += 1
+    assert refused

@@ -149,15 +149,15 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_f32_vec_kernel(const flo
 }
 
 // bf16 rows whose length is a multiple of 8: 16-byte loads, 8-byte stores;
-// rows of up to 4 * 8 * kBlock elements stay in registers between the two
+// rows of up to R * 8 * kBlock elements stay in registers between the two
 // passes, longer rows are read again (from L2).  Bound by memory: 2048 rows
 // of 4096 move 25 MB in 7.4 us at best (9.6 with a second read of the row).
-template <bool FP8>
+// R (16-byte chunks a thread keeps) is the least of 1, 2, 4 that holds a row.
+template <bool FP8, int R>
 __global__ __launch_bounds__(kBlock) void quant_per_row_bf16_vec_kernel(const uint16_t* __restrict__ src,
                                                                         uint8_t* __restrict__ dst,
                                                                         float* __restrict__ scales,
                                                                         int dim) {
-    constexpr int R = 4;  // 16-byte chunks a thread keeps
     const int64_t base = static_cast<int64_t>(blockIdx.x) * dim;
     const u32x4_t* s4 = reinterpret_cast<const u32x4_t*>(src + base);
     const int n8 = dim >> 3;
@@ -764,7 +764,10 @@ int quantize_per_row(const T* src, uint8_t* dst, float* scales, int rows, int di
                      (reinterpret_cast<uintptr_t>(dst) & 7) == 0;
     if constexpr (sizeof(T) == 2) {
         if (vec) {
-            quant_per_row_bf16_vec_kernel<FP8><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            if (dim <= 8 * kBlock) quant_per_row_bf16_vec_kernel<FP8, 1><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            else if (dim <= 16 * kBlock)
+                quant_per_row_bf16_vec_kernel<FP8, 2><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            else quant_per_row_bf16_vec_kernel<FP8, 4><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
             return check_launch(who);
         }
     } else {

@@ -1001,8 +1001,8 @@ __global__ __launch_bounds__(T == 1 ? 1024 : 512) void w4_decode_i8_kernel(W4Arg
 // ---------------------------------------------------------------------------
 // Tile kernel on 16x16x32 MFMAs: bf16 activations and output, asymmetric
 // int4 weights, several rows (plain, uniform batches, ragged groups), where
-// the 64- and 128-row 64 x 256 tiles (mma_tile_rs below) leave the chip idle
-// or have few rows.  A workgroup owns an output tile in one of the layouts
+// the 64 x 256 tile on 32x32x16 MFMAs (mma_tile32 below) leaves the chip idle
+// or has few rows.  A workgroup owns an output tile in one of the layouts
 // (L):
 //   L = 1:  16 RB x 256, waves wn = 0..3 on the same rows (RB = 1, 2: split-K
 //           launches and the fp32 interface);
@@ -1140,7 +1140,7 @@ __device__ __forceinline__ void store_bf16_block(const W4Args& p, uint16_t* C, c
 template <int BPS, bool GBIG, bool GR, bool SWI, int L, bool SK, int RB, bool F32>
 __device__ __forceinline__ void mma_tile(const W4Args& p, uint8_t* mm_lds, int bx, int by, int bz, int kb_in,
                                          int ke_in) {
-    static_assert(L >= 2 || SK || F32, "unsplit 64 x 256 bf16 tiles: mma_tile_rs");
+    static_assert(L >= 2 || SK || F32, "unsplit 64 x 256 bf16 tiles: mma_tile32");
     static_assert(RB == 4 || (RB <= 2 && !GR), "16- and 32-row blocks on plain launches");
     static_assert(!SK || (!GR && !SWI), "split-K on plain launches only");
     static_assert(L != 4 || SK, "the 8-wave 64 x 256 layout on split-K launches only");
@@ -1604,8 +1604,10 @@ __device__ __forceinline__ void mma_tile(const W4Args& p, uint8_t* mm_lds, int b
 }
 
 // ---------------------------------------------------------------------------
-// The fp32 interface's 64 x 256 tile on the 32x32x16 MFMA (W32 with F32:
-// layout 1, 64-row blocks; plain and split-K launches).  Same loads and LDS activation layout as mma_tile; what
+// The 64 x 256 tile on the 32x32x16 MFMA (W32: layout 1, 64-row blocks;
+// bf16 activations and output on plain, batched, grouped, SwiGLU, persistent
+// grouped and split-K launches, and the fp32 interface (F32) on plain and
+// split-K launches).  Same loads and LDS activation layout as mma_tile; what
 // changes is the matrix work per K tile and wave (64 rows x 64 columns x
 // 128 k):
 //   - the products run as 32 MFMAs of 32x32x16 instead of 64 of 16x16x32.
@@ -1626,7 +1628,9 @@ __device__ __forceinline__ void mma_tile(const W4Args& p, uint8_t* mm_lds, int b
 //     64 rows;
 //   - the wave's four column tiles nt0 + c form two 32-column blocks: block
 //     cb holds tile cb in lanes with (lane >> 4) & 1 == 0 and tile cb + 2 in
-//     the others;
+//     the others, so with SwiGLU's interleaved gate / up tiles block 0 holds
+//     the gates and block 1 the ups of the same two output tiles, in the
+//     same lanes;
 //   - MFMA q = (j, s) (k block j of 32, half s) takes in lane l the row /
 //     column l & 31 of the block and the 8 k at 32 j + 16 s + 8 (l >> 5):
 //     the weight dwords j of the prepacked tile's 16-byte chunk
@@ -1635,18 +1639,20 @@ __device__ __forceinline__ void mma_tile(const W4Args& p, uint8_t* mm_lds, int b
 //   - D element e of block (ib, cb) in lane l: row 32 ib + 8 (e >> 2) +
 //     4 (l >> 5) + (e & 3), column (lane & 15) of the lane's tile; the group
 //     correction acc += s * t uses one scale per lane and block.
-// The fp32 activations are staged in LDS (512 bytes per row); each wave splits
+// F32: fp32 activations staged in LDS (512 bytes per row); each wave splits
 // its own 16 rows into bf16 hi + lo in place before the rendezvous (with
 // their sums), and every product runs twice, hi and lo, as in mma_tile's
 // fp32 form; symmetric codes, fp32 scales, the alpha / beta epilogue.
 // Everything else (zero point folded into the codes, xs seeding each chain,
 // one correction per group, one K tile of loads in flight, unconditional
 // clamped loads) is as in mma_tile.
-template <bool GBIG, bool SK>
+template <bool GBIG, bool GR, bool SWI, bool PK, bool SK, bool F32>
 __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int bx, int by, int bz, int kb_in,
-                                           int ke_in) {
+                                           int ke_in, int pk_slot) {
+    static_assert(!SK || (!GR && !SWI && !PK), "split-K on plain launches only");
+    static_assert(!F32 || (!GR && !SWI && !PK), "the fp32 interface: plain launches");
     constexpr int BPS = 4;
-    constexpr int EA = 4;                         // activation bytes
+    constexpr int EA = F32 ? 4 : 2;               // activation bytes
     constexpr int RBYTES = kW4TileK * EA;         // LDS bytes per activation row
     constexpr int CPR = RBYTES / 16;              // 16-byte chunks per row
     constexpr int A_BYTES = 64 * RBYTES;          // one activation buffer
@@ -1659,10 +1665,31 @@ __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int
     const int kb = SK ? bz * p.kps : kb_in;
     const int ke = SK ? min(p.Kt, kb + p.kps) : ke_in;
     const int z = SK ? 0 : bz;
-    const int m0 = by * 64, m_end = p.M;
-    const uint8_t* const qw = p.qw + z * p.qw_bs;
-    const float* const Af = static_cast<const float*>(p.A) + z * p.a_bs;
-    const float* const scf = static_cast<const float*>(p.scales) + z * p.s_bs;
+    int m0, m_end;
+    const uint8_t* qw;
+    const uint16_t* sc;
+    const uint32_t* zs;
+    if constexpr (GR) {
+        int e;
+        if (!resolve_group<64>(p, by, e, m0, m_end)) return;  // uniform per workgroup
+        qw = p.qws[e];
+        sc = static_cast<const uint16_t*>(p.scs[e]);
+        zs = p.zss[e];
+        if constexpr (PK) {
+            qw = uniform_ptr(qw);
+            sc = uniform_ptr(sc);
+            zs = uniform_ptr(zs);
+        }
+    } else {
+        m0 = by * 64;
+        m_end = p.M;
+        qw = p.qw + z * p.qw_bs;
+        sc = static_cast<const uint16_t*>(p.scales) + z * p.s_bs;
+        zs = p.zeros + z * p.z_bs;
+    }
+    const uint16_t* A = static_cast<const uint16_t*>(p.A) + (GR ? 0 : z * p.a_bs);
+    const float* Af = static_cast<const float*>(p.A) + z * p.a_bs;
+    const float* scf = static_cast<const float*>(p.scales) + z * p.s_bs;
     uint32_t a_voff[DMA];  // as in mma_tile: LDS row idx / CPR, slot idx % CPR
 #pragma unroll
     for (int q = 0; q < DMA; ++q) {
@@ -1672,32 +1699,41 @@ __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int
         a_voff[q] = (static_cast<uint32_t>(row - m0) * static_cast<uint32_t>(p.K) +
                      static_cast<uint32_t>((slot ^ (r & 15)) * (16 / EA))) * EA;
     }
+    const uint32_t s_half = 16u * (col & 1);
     const int nt0 = min(bx * 4 * MM_CT + wave * MM_CT, p.Nt - 1);
     const int nt_left = p.Nt - nt0;
     auto extent = [](int64_t bytes) {
         return static_cast<int>(static_cast<uint32_t>(bytes < int64_t{0xFFFFFFFF} ? bytes : int64_t{0xFFFFFFFF}));
     };
+    constexpr int ES = F32 ? 4 : 2;  // scale bytes
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(qw) + static_cast<int64_t>(nt0) * p.Kt * kW4TileBytes, 0,
         extent(static_cast<int64_t>(nt_left) * p.Kt * kW4TileBytes), kBufWord3);
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(scf) + static_cast<int64_t>(nt0) * p.NG * 16, 0,
-                                          extent(static_cast<int64_t>(nt_left) * p.NG * 16 * 4), kBufWord3);
-    const __amdgpu_buffer_rsrc_t ra_ =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Af) + static_cast<int64_t>(m0) * p.K, 0,
-                                          extent(static_cast<int64_t>(m_end - m0) * p.K * EA), kBufWord3);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        F32 ? static_cast<void*>(const_cast<float*>(scf) + static_cast<int64_t>(nt0) * p.NG * 16)
+            : static_cast<void*>(const_cast<uint16_t*>(sc) + static_cast<int64_t>(nt0) * p.NG * 16),
+        0, extent(static_cast<int64_t>(nt_left) * p.NG * 16 * ES), kBufWord3);
+    const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(zs) + static_cast<int64_t>(nt0) * p.NG8 * 16, 0,
+        extent(F32 ? 0 : static_cast<int64_t>(nt_left) * p.NG8 * 16 * 4), kBufWord3);
+    const __amdgpu_buffer_rsrc_t ra_ = __builtin_amdgcn_make_buffer_rsrc(
+        F32 ? static_cast<void*>(const_cast<float*>(Af) + static_cast<int64_t>(m0) * p.K)
+            : static_cast<void*>(const_cast<uint16_t*>(A) + static_cast<int64_t>(m0) * p.K),
+        0, extent(static_cast<int64_t>(m_end - m0) * p.K * EA), kBufWord3);
     // the lane's tile in block cb (tiles past Nt re-read the last one)
-    uint32_t w_voff[2], s_voff[2];
+    uint32_t w_voff[2], s_voff[2], z_voff[2];
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
         const uint32_t dt = static_cast<uint32_t>(min(nt0 + cb + 2 * u, p.Nt - 1) - nt0);
         w_voff[cb] = dt * static_cast<uint32_t>(p.Kt) * kW4TileBytes + col * 16 + 256 * h;
-        s_voff[cb] = (dt * static_cast<uint32_t>(p.NG) * 16 + col) * 4;
+        s_voff[cb] = (dt * static_cast<uint32_t>(p.NG) * 16 + (F32 ? col : (col & ~1))) * ES;
+        z_voff[cb] = (dt * static_cast<uint32_t>(p.NG8) * 16 + col) * 4;
     }
 
     struct Regs {
         u32x4_t w[2][2];  // block cb, half s
         uint32_t sw[2];
+        uint32_t zw[2];
     };
     auto issue = [&](uint8_t* buf, Regs& R, int kt_in) {
         const int kt = min(kt_in + kb, p.Kt - 1);
@@ -1708,7 +1744,8 @@ __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int
         const int g = group_of_c<BPS, GBIG>(kt, 0, p.gmul);
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
-            R.sw[cb] = __builtin_amdgcn_raw_buffer_load_b32(rs, s_voff[cb], g * 16 * 4, 0);
+            if constexpr (!F32) R.zw[cb] = __builtin_amdgcn_raw_buffer_load_b32(rz, z_voff[cb], (g >> 3) * 16 * 4, 0);
+            R.sw[cb] = __builtin_amdgcn_raw_buffer_load_b32(rs, s_voff[cb], g * 16 * ES, 0);
 #pragma unroll
             for (int s = 0; s < 2; ++s)
                 R.w[cb][s] = __builtin_amdgcn_raw_buffer_load_b128(rw, w_voff[cb] + 512 * s, kt * kW4TileBytes, 0);
@@ -1753,36 +1790,53 @@ __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int
         f32x4_t xs = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            uint8_t* const c_hi = chunk_at(buf, row, 8 * j + 2 * (lane >> 4));
-            uint8_t* const c_lo = chunk_at(buf, row, 8 * j + 2 * (lane >> 4) + 1);
-            const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(c_hi);
-            const f32x4_t x1 = *reinterpret_cast<const f32x4_t*>(c_lo);
-            const float v[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-            u32x4_t ah, al;
+            if constexpr (F32) {
+                uint8_t* const c_hi = chunk_at(buf, row, 8 * j + 2 * (lane >> 4));
+                uint8_t* const c_lo = chunk_at(buf, row, 8 * j + 2 * (lane >> 4) + 1);
+                const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(c_hi);
+                const f32x4_t x1 = *reinterpret_cast<const f32x4_t*>(c_lo);
+                const float v[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+                u32x4_t ah, al;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint16_t h0 = f32_to_bf16(v[2 * e]), h1 = f32_to_bf16(v[2 * e + 1]);
-                ah[e] = static_cast<uint32_t>(h0) | (static_cast<uint32_t>(h1) << 16);
-                al[e] = pack_bf16x2(v[2 * e] - bf16_to_f32(h0), v[2 * e + 1] - bf16_to_f32(h1));
+                for (int e = 0; e < 4; ++e) {
+                    const uint16_t h0 = f32_to_bf16(v[2 * e]), h1 = f32_to_bf16(v[2 * e + 1]);
+                    ah[e] = static_cast<uint32_t>(h0) | (static_cast<uint32_t>(h1) << 16);
+                    al[e] = pack_bf16x2(v[2 * e] - bf16_to_f32(h0), v[2 * e + 1] - bf16_to_f32(h1));
+                }
+                *reinterpret_cast<u32x4_t*>(c_hi) = ah;
+                *reinterpret_cast<u32x4_t*>(c_lo) = al;
+                xs = mfma_bf16_16x16x32(ah, m144, xs);
+                xs = mfma_bf16_16x16x32(al, m144, xs);
+            } else {
+                xs = mfma_bf16_16x16x32(
+                    *reinterpret_cast<const u32x4_t*>(chunk_at(buf, row, 4 * j + (lane >> 4))), m144, xs);
             }
-            *reinterpret_cast<u32x4_t*>(c_hi) = ah;
-            *reinterpret_cast<u32x4_t*>(c_lo) = al;
-            xs = mfma_bf16_16x16x32(ah, m144, xs);
-            xs = mfma_bf16_16x16x32(al, m144, xs);
         }
         if (col == 0) *reinterpret_cast<f32x4_t*>(xs_l + 64 * (kt_in & 1) + 16 * wave + 4 * (lane >> 4)) = xs;
     };
     auto compute = [&](const uint8_t* buf, const Regs& R, int kt_in) {
         if (!live) return;
+        const int g = group_of_c<BPS, GBIG>(kb + kt_in, 0, p.gmul);
         const float* const xs_t = xs_l + 64 * (kt_in & 1);
-        const float scs[2] = {__uint_as_float(R.sw[0]), __uint_as_float(R.sw[1])};
-        // activation fragments of row block ib for k step q (the hi and the
-        // lo halves), read ahead of their use
-        constexpr int NH = 2;  // fragments per row block and k step
-        constexpr int RING = 2;
+        uint32_t zb[2];
+        float scs[2];
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+            if constexpr (F32) {
+                zb[cb] = 0x08080808u;  // symmetric codes: 16 - 8 in every byte
+                scs[cb] = __uint_as_float(R.sw[cb]);
+            } else {
+                zb[cb] = __builtin_amdgcn_perm(0u, 16u - ((R.zw[cb] >> (4 * (g & 7))) & 15u), 0u);
+                scs[cb] = f16_to_f32(static_cast<uint16_t>(R.sw[cb] >> s_half));
+            }
+        }
+        // activation fragment(s) of row block ib for k step q (F32: the hi
+        // and the lo halves), read ahead of their use
+        constexpr int NH = F32 ? 2 : 1;  // fragments per row block and k step
+        constexpr int RING = F32 ? 2 : 3;
         auto frag32 = [&](int q, int ib, int hh) {
             const int j = q >> 1, s = q & 1;
-            const int c = 8 * j + 2 * (2 * s + h) + hh;
+            const int c = F32 ? 8 * j + 2 * (2 * s + h) + hh : 4 * j + 2 * s + h;
             return *reinterpret_cast<const u32x4_t*>(chunk_at(buf, 32 * ib + (lane & 31), c));
         };
         u32x4_t af[RING][2][NH];
@@ -1817,7 +1871,7 @@ __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int
                     for (int hh = 0; hh < NH; ++hh) af[(q + RING - 1) % RING][ib][hh] = frag32(q + RING - 1, ib, hh);
             u32x4_t bq[2];
 #pragma unroll
-            for (int cb = 0; cb < 2; ++cb) bq[cb] = w4_operand_z(R.w[cb][s][j], 0x08080808u);  // symmetric codes: 16 - 8 in every byte
+            for (int cb = 0; cb < 2; ++cb) bq[cb] = w4_operand_z(R.w[cb][s][j], zb[cb]);
 #pragma unroll
             for (int ib = 0; ib < 2; ++ib)
 #pragma unroll
@@ -1871,6 +1925,24 @@ __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     const int ntw = bx * 4 * MM_CT + wave * MM_CT;  // the wave's first column tile
+    if constexpr (PK) {
+        if (pk_slot >= 0) {
+            // a K segment of a split tile: its partial sums in register
+            // order (f32x4 (ib, cb, e >> 2) of each lane), every row
+            f32x4_t* const W = reinterpret_cast<f32x4_t*>(p.ws) + static_cast<int64_t>(pk_slot) * kPkTileVecs +
+                               wave * 16 * 64 + lane;
+#pragma unroll
+            for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                    for (int i4 = 0; i4 < 4; ++i4)
+                        W[((ib * 2 + cb) * 4 + i4) * 64] =
+                            f32x4_t{acc[ib][cb][4 * i4], acc[ib][cb][4 * i4 + 1], acc[ib][cb][4 * i4 + 2],
+                                    acc[ib][cb][4 * i4 + 3]};
+            return;
+        }
+    }
     if constexpr (SK) {
         // the split's fp32 partial sums, ws[split][M][N]
         float* const W = p.ws + static_cast<int64_t>(bz) * p.M * p.N;
@@ -1889,385 +1961,42 @@ __device__ __forceinline__ void mma_tile32(const W4Args& p, uint8_t* mm_lds, int
         }
         return;
     }
-    // the reference's alpha / beta epilogue on fp32 C
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-        const int nt = ntw + cb + 2 * u;
-        const int cn = nt * kW4TileN + col;
-        if (nt >= p.Nt || cn >= p.N) continue;
-#pragma unroll
-        for (int ib = 0; ib < 2; ++ib)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = m0 + 32 * ib + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (row < m_end)
-                    w4_store<true>(p, z * p.c_bs + static_cast<int64_t>(row) * p.N + cn, acc[ib][cb][e]);
-            }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// The bf16 tile on the 32x32x16 MFMA: 32 IB rows x 256 columns per
-// workgroup, four waves of 32 IB rows x 64 columns (bf16 activations and
-// output on plain, batched, grouped, SwiGLU, persistent grouped and split-K
-// launches).  IB = 2 is the 64-row tile; IB = 4 (128 rows) serves plain
-// launches with rows enough (launch_mma).
-//
-// What bounds it is issuing the weight decode and the group corrections
-// beside the MFMAs, and the power all three draw: the chip holds 1.7-1.9 GHz
-// under this load.  So the accumulators are kept in units of the current
-// group's scale,
-//     acc_g = acc_{g-1} * (s_{g-1} / s_g) - 144 sum_k x + sum_k x (144 + u - z),
-// and multiplied by the last scale at the end: one FMA per element and K
-// tile both rescales and seeds the tile's sums (an accumulator and a separate
-// chain per group took the FMA, a copied seed and twice the registers).  The
-// registers this frees hold 128 rows per wave at two waves per SIMD, which
-// decodes each weight once per 128 rows instead of 64: 5.2 VALU instructions
-// per MFMA instead of 6.4.
-// M=4096, K=8192, N=28672 (us, one box): 1,810 in the earlier 64-row form,
-// 1,765 with IB = 2, 1,603 with IB = 4 (1,200 TFLOP/s; MFMA pipe 65% busy,
-// 57% before); a library bf16 GEMM of that shape takes 1,325.
-//   - Ratio: rcp and one Newton step (within 1 ulp of s_{g-1} / s_g, exactly
-//     1 for equal scales).  A zero scale keeps the unit and zeroes the
-//     group's (u - z); a non-finite one propagates as the product would.
-//   - Loads: activations by DMA into one of two LDS buffers a K tile ahead
-//     (16-byte chunk c of row r in slot c ^ (r & 15)); weights in registers,
-//     each half reloaded as soon as its last operand is decoded.
-//   - The activation sums -144 sum_k x are made once per workgroup: each
-//     wave sums the 8 IB rows that its own DMAs carried (MFMAs of 16x16x32
-//     against -144) at k step 6 of the tile before, where they are long
-//     there (vmcnt(6): six later loads), and the rendezvous that opens the
-//     tile hands them to every wave through LDS.
-//   - The wave's four column tiles nt0 + c form two 32-column blocks: block
-//     cb holds tile cb in lanes with (lane >> 4) & 1 == 0 and tile cb + 2 in
-//     the others, so with SwiGLU's interleaved gate / up tiles block 0 holds
-//     the gates and block 1 the ups of the same two output tiles, in the
-//     same lanes.
-//   - MFMA (q, ib, cb), k step q = (half s = q >> 2, k block j = q & 3),
-//     takes in lane l the row / column l & 31 and the 8 k at 32 j + 16 s +
-//     8 (l >> 5): dword j of the prepacked tile's 16-byte chunk (l & 15) +
-//     16 (l >> 5) + 32 s, and LDS chunk 4 j + 2 s + (l >> 5).  Weight
-//     operands are decoded one k step ahead, fragments read four MFMA pairs
-//     ahead.
-//   - D element e of block (ib, cb) in lane l: row 32 ib + 8 (e >> 2) +
-//     4 (l >> 5) + (e & 3), column (lane & 15) of the lane's tile.
-//   - s_setprio: the products run at raised priority, so the other wave of
-//     the SIMD does its FMAs under them (IB = 4: 2.3%; IB = 2, MoE layers of
-//     512 and 300 tokens: 1.8% and 0.5%).
-//   - On persistent grouped launches this form is still behind the one with a
-//     chain per group: MoE layers of 512 / 300 tokens 0.9% / 1.6% longer.
-// Every load is unconditional (rows past the end read the last row; column
-// tiles past Nt re-read the last one; the K tile past the end is the last
-// one again and is never used).  Requires K % 128 == 0.
-// SK, PK, pk_slot: as for mma_tile.
-template <bool GBIG, bool GR, bool SWI, bool PK, bool SK, int IB>
-__device__ __forceinline__ void mma_tile_rs(const W4Args& p, uint8_t* mm_lds, int bx, int by, int bz, int kb_in,
-                                            int ke_in, int pk_slot) {
-    static_assert(!SK || (!GR && !SWI && !PK), "split-K on plain launches only");
-    constexpr int BPS = 4;
-    constexpr int ROWS = 32 * IB;
-    constexpr int RBYTES = kW4TileK * 2;          // LDS bytes per activation row
-    constexpr int A_BYTES = ROWS * RBYTES;        // one activation buffer
-    constexpr int DMA = A_BYTES / 1024 / 4;       // activation DMAs per wave per K tile
-    constexpr int SB = IB / 2;                    // 16-row blocks a wave sums
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int col = lane & 15, h = lane >> 5, u = (lane >> 4) & 1;
-    const int kb = SK ? bz * p.kps : kb_in;
-    const int ke = SK ? min(p.Kt, kb + p.kps) : ke_in;
-    const int z = SK ? 0 : bz;
-    int m0, m_end;
-    const uint8_t* qw;
-    const uint16_t* sc;
-    const uint32_t* zs;
-    if constexpr (GR) {
-        int e;
-        if (!resolve_group<ROWS>(p, by, e, m0, m_end)) return;  // uniform per workgroup
-        qw = p.qws[e];
-        sc = static_cast<const uint16_t*>(p.scs[e]);
-        zs = p.zss[e];
-        if constexpr (PK) {
-            qw = uniform_ptr(qw);
-            sc = uniform_ptr(sc);
-            zs = uniform_ptr(zs);
-        }
-    } else {
-        m0 = by * ROWS;
-        m_end = p.M;
-        qw = p.qw + z * p.qw_bs;
-        sc = static_cast<const uint16_t*>(p.scales) + z * p.s_bs;
-        zs = p.zeros + z * p.z_bs;
-    }
-    const uint16_t* A = static_cast<const uint16_t*>(p.A) + (GR ? 0 : z * p.a_bs);
-    uint32_t a_voff[DMA];  // LDS row idx / 16, slot idx % 16
-#pragma unroll
-    for (int q = 0; q < DMA; ++q) {
-        const int idx = (DMA * wave + q) * 64 + lane;
-        const int r = idx >> 4, slot = idx & 15;
-        const int row = min(m0 + r, m_end - 1);
-        a_voff[q] = (static_cast<uint32_t>(row - m0) * static_cast<uint32_t>(p.K) +
-                     static_cast<uint32_t>((slot ^ (r & 15)) * 8)) * 2;
-    }
-    const uint32_t s_half = 16u * (col & 1);
-    const int nt0 = min(bx * 4 * MM_CT + wave * MM_CT, p.Nt - 1);
-    const int nt_left = p.Nt - nt0;
-    auto extent = [](int64_t bytes) {
-        return static_cast<int>(static_cast<uint32_t>(bytes < int64_t{0xFFFFFFFF} ? bytes : int64_t{0xFFFFFFFF}));
-    };
-    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(qw) + static_cast<int64_t>(nt0) * p.Kt * kW4TileBytes, 0,
-        extent(static_cast<int64_t>(nt_left) * p.Kt * kW4TileBytes), kBufWord3);
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(sc) + static_cast<int64_t>(nt0) * p.NG * 16, 0,
-        extent(static_cast<int64_t>(nt_left) * p.NG * 16 * 2), kBufWord3);
-    const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint32_t*>(zs) + static_cast<int64_t>(nt0) * p.NG8 * 16, 0,
-        extent(static_cast<int64_t>(nt_left) * p.NG8 * 16 * 4), kBufWord3);
-    const __amdgpu_buffer_rsrc_t ra_ = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(A) + static_cast<int64_t>(m0) * p.K, 0,
-        extent(static_cast<int64_t>(m_end - m0) * p.K * 2), kBufWord3);
-    uint32_t w_voff[2], s_voff[2], z_voff[2];
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-        const uint32_t dt = static_cast<uint32_t>(min(nt0 + cb + 2 * u, p.Nt - 1) - nt0);
-        w_voff[cb] = dt * static_cast<uint32_t>(p.Kt) * kW4TileBytes + col * 16 + 256 * h;
-        s_voff[cb] = (dt * static_cast<uint32_t>(p.NG) * 16 + (col & ~1)) * 2;
-        z_voff[cb] = (dt * static_cast<uint32_t>(p.NG8) * 16 + col) * 4;
-    }
-
-    // the K tile in use: weights of block cb, half s; each half's registers
-    // are reloaded with the next tile's as soon as its products are issued
-    u32x4_t w[2][2];
-    uint32_t sw[2], zw[2];
-    auto issue_a = [&](uint32_t buf, int kt_in) {
-        const int kt = min(kt_in + kb, p.Kt - 1);
-#pragma unroll
-        for (int q = 0; q < DMA; ++q)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra_, (LHQ_LDS_AS void*)(mm_lds + buf + (DMA * wave + q) * 1024), 16,
-                                                     a_voff[q], kt * kW4TileK * 2, 0, 0);
-    };
-    auto issue_sz = [&](int kt_in) {
-        const int kt = min(kt_in + kb, p.Kt - 1);
-        const int g = group_of_c<BPS, GBIG>(kt, 0, p.gmul);
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-            zw[cb] = __builtin_amdgcn_raw_buffer_load_b32(rz, z_voff[cb], (g >> 3) * 16 * 4, 0);
-            sw[cb] = __builtin_amdgcn_raw_buffer_load_b32(rs, s_voff[cb], g * 16 * 2, 0);
-        }
-    };
-    auto issue_w = [&](int kt_in, int s) {
-        const int kt = min(kt_in + kb, p.Kt - 1);
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-            w[cb][s] = __builtin_amdgcn_raw_buffer_load_b128(rw, w_voff[cb] + 512 * s, kt * kW4TileBytes, 0);
-    };
-
-    f32x16_t acc[IB][2];
-#pragma unroll
-    for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[ib][cb][e] = 0.f;
-    float unit[2] = {0.f, 0.f};  // the scale that acc[.][cb] is in units of
-    // fragment chunk 4 j + 2 s + h of row l & 31, and chunk 4 j + (lane >> 4)
-    // of the 16-row block the wave sums: their slots differ from these by
-    // XORs of constants
-    const uint32_t lane_f = (lane & 31) * RBYTES + ((h ^ (lane & 15)) * 16);
-    const uint32_t lane_s = (16 * SB * wave + col) * RBYTES + (((lane >> 4) ^ col) * 16);
-    auto sums = [&](uint32_t buf, int kt_in) {
-        asm volatile("" ::: "memory");
-        uint32_t sbase = buf + lane_s;
-        asm volatile("" : "+v"(sbase));
-        uint32_t m = kM144Bf16x2;
-        asm volatile("" : "+v"(m));  // (four registers only here)
-        const u32x4_t m144 = {m, m, m, m};
-        uint32_t xbase = 2 * A_BYTES + 4 * ROWS * (kt_in & 1) + 64 * SB * wave + 16 * (lane >> 4);
-        asm volatile("" : "+v"(xbase));
-        f32x4_t xs[SB];
-#pragma unroll
-        for (int b = 0; b < SB; ++b) xs[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int b = 0; b < SB; ++b)
-                xs[b] = mfma_bf16_16x16x32(
-                    *reinterpret_cast<const u32x4_t*>(mm_lds + (sbase ^ (64 * j)) + 16 * RBYTES * b), m144, xs[b]);
-        if (col == 0)
-#pragma unroll
-            for (int b = 0; b < SB; ++b) *reinterpret_cast<f32x4_t*>(mm_lds + xbase + 64 * b) = xs[b];
-    };
-    auto compute = [&](uint32_t buf, int kt_in) {
-        const int g = group_of_c<BPS, GBIG>(min(kb + kt_in, p.Kt - 1), 0, p.gmul);
-        uint32_t xbase = 2 * A_BYTES + 4 * ROWS * (kt_in & 1) + 16 * h;
-        asm volatile("" : "+v"(xbase));
-        uint32_t zb[2], lowm[2];
-        float ratio[2];
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-            const float s = f16_to_f32(static_cast<uint16_t>(sw[cb] >> s_half));
-            const bool none = s == 0.0f;
-            const float s1 = none ? unit[cb] : s;
-            zb[cb] = none ? 0x10101010u : __builtin_amdgcn_perm(0u, 16u - ((zw[cb] >> (4 * (g & 7))) & 15u), 0u);
-            lowm[cb] = none ? 0u : 0x0F0F0F0Fu;
-            const float rc = __builtin_amdgcn_rcpf(s1);
-            const float r0 = unit[cb] * rc;
-            const float r1 = __builtin_fmaf(__builtin_fmaf(-s1, r0, unit[cb]), rc, r0);
-            ratio[cb] = s1 == unit[cb] ? 1.0f : fabsf(r1) < __builtin_inff() ? r1 : r0;
-            unit[cb] = s1;
-        }
-        issue_sz(kt_in + 1);
-        // step t = (q, ib): the fragment of row block ib, k step q = (s, j)
-        uint32_t fbase = buf + lane_f;
-        // opaque, so that the eight addresses derived from it are not kept in
-        // registers across K tiles
-        asm volatile("" : "+v"(fbase));
-        auto frag = [&](int t) {
-            const int q = t / IB, ib = t % IB;
-            const uint32_t c = 4 * (q & 3) + 2 * (q >> 2);
-            return *reinterpret_cast<const u32x4_t*>(mm_lds + (fbase ^ (c * 16)) + 32 * RBYTES * ib);
-        };
-        auto operand = [&](uint32_t d, int cb) {
-            const uint32_t lo = (d & lowm[cb]) + zb[cb];
-            const uint32_t hi = ((d >> 4) & lowm[cb]) + zb[cb];
-            constexpr uint32_t kExp = 0x43434343u;
-            return u32x4_t{__builtin_amdgcn_perm(kExp, lo, 0x04010400u), __builtin_amdgcn_perm(kExp, lo, 0x04030402u),
-                           __builtin_amdgcn_perm(kExp, hi, 0x04010400u), __builtin_amdgcn_perm(kExp, hi, 0x04030402u)};
-        };
-        constexpr int RING = 5;
-        u32x4_t af[RING];
-#pragma unroll
-        for (int t = 0; t < RING - 1; ++t) af[t] = frag(t);
-        f32x4_t x[2][4];
-        auto seeds = [&](int ib) {
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4)
-                x[ib & 1][i4] = *reinterpret_cast<const f32x4_t*>(mm_lds + xbase + 128 * ib + 32 * i4);
-        };
-        seeds(0);
-#pragma unroll
-        for (int ib = 0; ib < IB; ++ib) {
-            if (ib + 1 < IB) seeds(ib + 1);
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-#pragma unroll
-                for (int cb = 0; cb < 2; ++cb)
-                    acc[ib][cb][e] = __builtin_fmaf(acc[ib][cb][e], ratio[cb], x[ib & 1][e >> 2][e & 3]);
-            // the sums stay live past their last use: added to in place, their
-            // registers would become the accumulators' (and be copied back
-            // every K tile)
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) asm volatile("" ::"v"(x[ib & 1][i4]));
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __builtin_amdgcn_s_setprio(1);
-        u32x4_t bq[2][2];
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) bq[0][cb] = operand(w[cb][0][0], cb);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            if (q + 1 < 8)
-#pragma unroll
-                for (int cb = 0; cb < 2; ++cb) bq[(q + 1) & 1][cb] = operand(w[cb][(q + 1) >> 2][(q + 1) & 3], cb);
-            if (q == 3) issue_w(kt_in + 1, 0);
-            if (q == 7) issue_w(kt_in + 1, 1);
-            if (q == 6) {
-                // vmcnt(6): the activation DMAs of the next tile (the scales,
-                // zeros and half 0 of the weights, six loads, came later)
-                __builtin_amdgcn_s_waitcnt(0x0F76);
-                sums(A_BYTES - buf, kt_in + 1);
-            }
-#pragma unroll
-            for (int ib = 0; ib < IB; ++ib) {
-                const int t = q * IB + ib;
-                if (t + RING - 1 < 8 * IB) af[(t + RING - 1) % RING] = frag(t + RING - 1);
-#pragma unroll
-                for (int cb = 0; cb < 2; ++cb)
-                    acc[ib][cb] = mfma_bf16_32x32x16(af[t % RING], bq[q & 1][cb], acc[ib][cb]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __builtin_amdgcn_s_setprio(0);
-    };
-    auto rendezvous = [&]() {
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    };
-
-    const int kh = ke - kb;
-    issue_a(0, 0);
-    issue_sz(0);
-    issue_w(0, 0);
-    issue_w(0, 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    sums(0, 0);
-    for (int kt = 0; kt < kh; ++kt) {
-        const uint32_t cur = (kt & 1) * A_BYTES;
-        rendezvous();
-        issue_a(A_BYTES - cur, kt + 1);  // clamped past the end: never used
-        __builtin_amdgcn_sched_barrier(0);  // the wait at k step 6 counts the loads that follow
-        compute(cur, kt);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[ib][cb][e] *= unit[cb];
-
-    const int ntw = bx * 4 * MM_CT + wave * MM_CT;  // the wave's first column tile
-    if constexpr (PK) {
-        if (pk_slot >= 0) {
-            f32x4_t* const W = reinterpret_cast<f32x4_t*>(p.ws) + static_cast<int64_t>(pk_slot) * kPkTileVecs * (IB / 2) +
-                               wave * 8 * IB * 64 + lane;
-#pragma unroll
-            for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-                for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-                    for (int i4 = 0; i4 < 4; ++i4)
-                        W[((ib * 2 + cb) * 4 + i4) * 64] =
-                            f32x4_t{acc[ib][cb][4 * i4], acc[ib][cb][4 * i4 + 1], acc[ib][cb][4 * i4 + 2],
-                                    acc[ib][cb][4 * i4 + 3]};
-            return;
-        }
-    }
-    if constexpr (SK) {
-        float* const W = p.ws + static_cast<int64_t>(bz) * p.M * p.N;
+    if constexpr (F32) {
+        // the reference's alpha / beta epilogue on fp32 C
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
             const int nt = ntw + cb + 2 * u;
             const int cn = nt * kW4TileN + col;
             if (nt >= p.Nt || cn >= p.N) continue;
 #pragma unroll
-            for (int ib = 0; ib < IB; ++ib)
+            for (int ib = 0; ib < 2; ++ib)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const int row = m0 + 32 * ib + 8 * (e >> 2) + 4 * h + (e & 3);
-                    if (row < m_end) W[static_cast<int64_t>(row) * p.N + cn] = acc[ib][cb][e];
+                    if (row < m_end)
+                        w4_store<true>(p, z * p.c_bs + static_cast<int64_t>(row) * p.N + cn, acc[ib][cb][e]);
                 }
         }
-        return;
-    }
-    uint16_t* const C = static_cast<uint16_t*>(p.C) + (GR ? 0 : z * p.c_bs);
+    } else {
+        uint16_t* const C = static_cast<uint16_t*>(p.C) + (GR ? 0 : z * p.c_bs);
 #pragma unroll
-    for (int cb = 0; cb < (SWI ? 1 : 2); ++cb) {
-        const int nt = ntw + cb + 2 * u;
-        const int cn = (SWI ? (ntw >> 1) + u : nt) * kW4TileN + col;
-        if (nt >= p.Nt || cn >= p.N) continue;
+        for (int cb = 0; cb < (SWI ? 1 : 2); ++cb) {
+            // SwiGLU: block 0 holds the gates, block 1 the ups of output tile
+            // ntw / 2 + u
+            const int nt = ntw + cb + 2 * u;
+            const int cn = (SWI ? (ntw >> 1) + u : nt) * kW4TileN + col;
+            if (nt >= p.Nt || cn >= p.N) continue;
 #pragma unroll
-        for (int ib = 0; ib < IB; ++ib)
+            for (int ib = 0; ib < 2; ++ib)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = m0 + 32 * ib + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (row >= m_end) continue;
-                if constexpr (SWI)
-                    C[static_cast<int64_t>(row) * p.N + cn] = f32_to_bf16(swiglu(acc[ib][0][e], acc[ib][1][e]));
-                else C[static_cast<int64_t>(row) * p.N + cn] = f32_to_bf16(acc[ib][cb][e]);
-            }
+                for (int e = 0; e < 16; ++e) {
+                    const int row = m0 + 32 * ib + 8 * (e >> 2) + 4 * h + (e & 3);
+                    if (row >= m_end) continue;
+                    if constexpr (SWI)
+                        C[static_cast<int64_t>(row) * p.N + cn] = f32_to_bf16(swiglu(acc[ib][0][e], acc[ib][1][e]));
+                    else C[static_cast<int64_t>(row) * p.N + cn] = f32_to_bf16(acc[ib][cb][e]);
+                }
+        }
     }
 }
 
@@ -2293,11 +2022,10 @@ __device__ __forceinline__ void mma_tile_rs(const W4Args& p, uint8_t* mm_lds, in
 template <int BPS, bool GBIG, bool GR, bool SWI, int L, bool SK = false, int RB = 4, bool F32 = false, bool PK = false,
           bool W32 = false>
 __global__ __launch_bounds__(L >= 3 ? 512 : 256, L == 3 ? 1 : 2) void w4_mma_kernel(W4Args p) {
-    static_assert(!W32 || (BPS == 4 && L == 1 && (RB == 4 || (RB == 8 && !F32 && !PK))), "the 32x32x16 tiles");
+    static_assert(!W32 || (BPS == 4 && L == 1 && RB == 4), "the 32x32x16 tile: 64 x 256 tiles");
     extern __shared__ __attribute__((aligned(1024))) uint8_t mm_lds[];
     auto tile = [&](int bx, int by, int bz, int k0, int k1, int slot) {
-        if constexpr (W32 && F32) mma_tile32<GBIG, SK>(p, mm_lds, bx, by, bz, k0, k1);
-        else if constexpr (W32) mma_tile_rs<GBIG, GR, SWI, PK, SK, RB / 2>(p, mm_lds, bx, by, bz, k0, k1, slot);
+        if constexpr (W32) mma_tile32<GBIG, GR, SWI, PK, SK, F32>(p, mm_lds, bx, by, bz, k0, k1, slot);
         else mma_tile<BPS, GBIG, GR, SWI, L, SK, RB, F32>(p, mm_lds, bx, by, bz, k0, k1);
     };
     if constexpr (!PK) {
@@ -2627,44 +2355,10 @@ int device_cus() {
     return cus;
 }
 
-// the 128-row tile of plain launches
-constexpr size_t kMma32BigLds = 2 * 128 * kW4TileK * 2 + 2 * 128 * 4;
-template <bool GBIG>
-void launch_mma32_big(const W4Args& a, unsigned batch, hipStream_t s) {
-    const dim3 grid(ceil_div(a.Nt, 4 * MM_CT), ceil_div(a.M, 128), batch);
-    allow_cu_lds<&w4_mma_kernel<4, GBIG, false, false, 1, false, 8, false, false, true>>();
-    w4_mma_kernel<4, GBIG, false, false, 1, false, 8, false, false, true><<<grid, 256, kMma32BigLds, s>>>(a);
-}
-// ... where it takes less time than the 64-row tile.  Two workgroups of
-// either fit a CU; with rounds of 2 per CU as the unit, a last round of at
-// most one per CU costs 0.63, and a 128-row round 1.73 of a 64-row one
-// (K=8192, N=28672: 448 workgroups of 128 rows 228 us, of 64 rows 132, 224 of
-// 128 rows 144).  That orders every shape measured (us, 64 / 128 rows):
-// K=8192, N=28672 M=512 254 / 228, 640 312 / 333, 768 364 / 342, 2048 922 /
-// 843, 4096 1,783 / 1,611; K=4096, N=11008 M=1300 132 / 115, 1536 156 / 171,
-// 4096 371 / 358; K=N=4096 M=3072 98 / 104, 4096 135 / 120.
-bool big_tiles(const W4Args& a, int batch) {
-    static const int env = tuning_knob("LHQ_W4_BIG", -1);
-    if (env >= 0) return env != 0;
-    const int64_t slots = 2 * std::max(device_cus(), 1), x = static_cast<int64_t>(ceil_div(a.Nt, 4 * MM_CT)) * batch;
-    auto rounds = [&](int rows) {
-        const int64_t w = x * ceil_div(a.M, rows), last = w % slots;
-        return static_cast<double>(w / slots) + (last == 0 ? 0.0 : 2 * last <= slots ? 0.63 : 1.0);
-    };
-    return 1.73 * rounds(128) < rounds(64);
-}
-
 template <bool GR, bool SWI, int L>
 void launch_mma_l(const W4Args& a, unsigned row_tiles, unsigned batch, hipStream_t s) {
     const dim3 grid(ceil_div(a.Nt, ((L == 1) ? 4 : 2) * MM_CT), row_tiles, batch);
     if constexpr (L == 1) {
-        if constexpr (!GR) {
-            if (big_tiles(a, static_cast<int>(batch))) {
-                if (a.gmul) launch_mma32_big<true>(a, batch, s);
-                else launch_mma32_big<false>(a, batch, s);
-                return;
-            }
-        }
         if (a.gmul) launch_mma32<true, GR, SWI, false>(a, grid, s);
         else launch_mma32<false, GR, SWI, false>(a, grid, s);
     } else {

@@ -1,11 +1,13 @@
-"""The 64- and 128-row bf16 tiles of the W4A16 prefill, whose accumulators are
-kept in units of the current group's scale: shapes on both sides of the choice
-between them with ragged last rows and columns, G = 128 and 256, batches, and
-scales that vary as far as fp16 goes, vanish or are all zero.
+"""The 64 x 256 bf16 tile of the W4A16 prefill on 32x32x16 MFMAs: shapes with
+ragged last rows and columns around its row count, G = 128 and 256, batches,
+and scales that vary as far as fp16 goes, vanish or are all zero, under
+ordinary and very large activations.
 
-Tolerance, against float64 on the same codes: a partial sum of a column never
-exceeds 303 sum_k s |x| (terms x (144 + u - z) and -144 x), and each of the
-K + 4 K/G additions, rescalings and products rounds once (2^-24), so
+Tolerance, against float64 on the same codes: inside a group a partial sum of a
+column never exceeds 303 sum_k |x| (terms x (144 + u - z) and -144 x), the
+group's sum is then multiplied by its scale (exactly 0 for a zero scale, so
+such a group adds nothing, rounding errors included) and added, and each of the
+K + 4 K/G additions and products rounds once (2^-24), so
 |error| <= 2^-24 (K + 4 K/G) 303 sum_k s |x|, plus half an ulp of bf16 (2^-8
 |want|).  Relative Frobenius: bf16 rounding alone is at most 2^-9, so 2.5e-3.
 """
@@ -48,8 +50,8 @@ def _check(got, x, u, z, s, G):
     return np.linalg.norm(got - want) / max(np.linalg.norm(want), 1e-300)
 
 
-# 128-row tiles: 4 x 113 and 4 x 112 workgroups; 64-row: 8 x 17, one row
-# tile, one past a tile
+# 8 row tiles at two widths, 7 with one row over, 8 x 17, one row tile, one
+# row past a tile
 @pytest.mark.parametrize("M,N,K,G", [(450, 28700, 256, 128), (512, 28672, 512, 256), (385, 28672, 128, 128),
                                      (449, 4100, 384, 128), (64, 20000, 256, 128), (65, 40000, 512, 256)])
 def test_shapes(oracle, ops, M, N, K, G):
@@ -93,7 +95,7 @@ def _hard_scales(NG, N, seed):
     return s
 
 
-# 64-row, 128-row and split-K launches of the tile
+# two row tiles, eight, and a split-K launch
 @pytest.mark.parametrize("M,N,K", [(80, 16400, 1024), (450, 28672, 1024), (64, 4096, 8192)])
 def test_scale_range(oracle, ops, M, N, K):
     G = 128
@@ -105,6 +107,23 @@ def test_scale_range(oracle, ops, M, N, K):
     xf = D.bf16_bits_to_f32(xb)
     _check(got, xf, u, z, s, G)
     assert (got[:, np.arange(N) % 8 == 2] == 0).all()
+
+
+# the same launches: groups of zero scale hold activations up to 1e8 times the
+# others'
+@pytest.mark.parametrize("M,N,K", [(80, 16400, 1024), (450, 28672, 1024), (64, 4096, 8192)])
+def test_zero_scaled_groups_add_nothing(oracle, ops, M, N, K):
+    G = 128
+    u, z, s, x = _case(M, N, K, G, K + 1)
+    g = D.rng(K)
+    dead = np.arange(K // G) % 3 == 1
+    s[dead] = 0
+    x *= np.where(dead, g.choice([1e6, 1e7, 1e8], K // G), 1.0).astype(np.float32).repeat(G)
+    xb = D.to_bf16_bits(oracle, x)
+    w = _prepack(ops, u, z, s, K, N, G)
+    C = ops.gemm_w4a16_bf16_ws(ops.dev(xb), w, ops.w4a16_bf16_workspace(M, w))
+    got = D.bf16_bits_to_f32(ops.host(C, np.uint16)).astype(np.float64)
+    assert _check(got, D.bf16_bits_to_f32(xb), u, z, s, G) <= 2.5e-3
 
 
 def test_non_finite_scales_and_rows(oracle, ops):

@@ -386,6 +386,13 @@ int lhq_gemm_f32_batched(const float* A, const float* B, float* C, int batch, in
  * reference's rule (dtypes.hpp:87-98).  counts: 2 device uint64, set to
  * {non-NaN mismatches, NaN mismatches}; both are 0 on a conforming device. */
 int lhq_selftest_bf16(unsigned long long* counts, void* stream);
+/* The form of the W4A16 kernel for a few rows (weights streamed, rows staged
+ * on chip) that this call takes on the current device with 16-byte aligned
+ * activations: 16 * (16-row blocks) + column tiles per workgroup, 0 where
+ * another kernel takes it.  f32 = 0: lhq_gemm_w4a16_bf16_ws and _noalloc;
+ * f32 != 0: lhq_gemm_w4a16 and _ws.  For tests, which assert the kernel they
+ * mean to run. */
+int lhq_selftest_w4_stream(int M, int N, int K, int G, int f32);
 /* The matrix-core rate probes bench.py uses are in the separate diagnostics
  * library (include/longhorn_diag.h, liblonghorn_diag.so). */
 

@@ -391,3 +391,16 @@ int launch_w4_stream(const W4Args& a, bool f32, int rb, hipStream_t s, const cha
 }
 
 }  // namespace lhq
+
+extern "C" int lhq_selftest_w4_stream(int M, int N, int K, int G, int f32) {
+    using namespace lhq;
+    if (M <= 0 || N <= 0 || K <= 0 || G <= 0) return 0;
+    W4Args a{};
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.G = G;
+    a.Nt = ceil_div(N, kW4TileN);
+    const int rb = w4_stream_rb(a, f32 != 0);
+    return rb ? 16 * rb + column_tiles(a, f32 != 0, rb, std::max(w4_device_cus(), 1)) : 0;
+}

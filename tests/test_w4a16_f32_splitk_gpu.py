@@ -61,9 +61,9 @@ def _run(ops, A, w, C0, alpha, beta, ws_bytes, fill=None):
     (5, 8192, 4104, 256, 0.5, 2.0),        # N % 16 != 0, G = 256, alpha / beta
     (16, 8192, 4096, 128, 1.0, 0.0),       # 16-row blocks
     (16, 2304, 16384, 384, -1.0, 1.0),     # G = 384: split boundaries inside scale groups
-    (17, 1024, 1040, 128, 1.0, 0.0),       # 32-row blocks, 17 live rows, ragged N
+    (17, 2176, 1040, 128, 1.0, 0.0),       # 32-row blocks, 17 live rows, ragged N
     (24, 4096, 2048, 128, 2.0, -0.5),
-    (32, 2048, 1000, 256, 1.0, 0.0),
+    (32, 2304, 1000, 256, 1.0, 0.0),
     (33, 1152, 512, 128, 1.0, 0.0),        # 64-row blocks, 33 live rows, 9 K tiles
     (48, 4096, 1024, 128, 1.0, 1.0),
     (64, 8192, 512, 128, 0.5, 0.0),        # config 5 K
@@ -75,14 +75,16 @@ def test_f32_splitk_matches_oracle(oracle, ops, M, K, N, G, alpha, beta):
     A, w, C0, want = _case(oracle, ops, M, K, N, G, seed=2100 + M + K // 128, alpha=alpha, beta=beta)
     n = _ws_bytes(ops, M, K, N, G)
     assert n > 0 and n % (M * N * 4) == 0 and n // (M * N * 4) >= 2   # split
+    assert ops.lib().lhq_selftest_w4_stream(M, N, K, G, 1) == 0  # the kernel that needs no split leaves it
     got = _run(ops, A, w, C0, alpha, beta, n, fill=0x7F)
     err = rel_frobenius(got, want)
     assert err <= TOL_F32, f"rel Frobenius {err:.3e}"
 
 
 def test_f32_splitk_beta0_ignores_nan_in_c(oracle, ops):
-    M, K, N, G = 24, 2048, 768, 128
+    M, K, N, G = 24, 2176, 768, 128
     A, w, _, want = _case(oracle, ops, M, K, N, G, seed=2300)
+    assert ops.lib().lhq_selftest_w4_stream(M, N, K, G, 1) == 0 and _ws_bytes(ops, M, K, N, G) > 0
     got = _run(ops, A, w, np.full((M, N), np.nan, np.float32), 1.0, 0.0, _ws_bytes(ops, M, K, N, G))
     assert np.isfinite(got).all()
     assert rel_frobenius(got, want) <= TOL_F32
@@ -95,6 +97,7 @@ def test_f32_splitk_deterministic_and_workspace_rules(oracle, ops):
     M, K, N, G = 32, 4096, 2048, 128
     A, w, C0, want = _case(oracle, ops, M, K, N, G, seed=2400, alpha=0.75, beta=0.5)
     n = _ws_bytes(ops, M, K, N, G)
+    assert n > 0 and ops.lib().lhq_selftest_w4_stream(M, N, K, G, 1) == 0
     outs = [_run(ops, A, w, C0, 0.75, 0.5, n, fill=f) for f in (0, 0xFF, 0x41)]
     assert all(np.array_equal(outs[0].view(np.uint32), o.view(np.uint32)) for o in outs[1:])
     small = _run(ops, A, w, C0, 0.75, 0.5, 2 * M * N * 4)   # room for two splits
@@ -139,7 +142,7 @@ def test_f32_splitk_in_a_captured_hip_graph(oracle, ops):
     M, K, N, G = 16, 8192, 4096, 128
     A, w, C0, _ = _case(oracle, ops, M, K, N, G, seed=2500, alpha=1.5, beta=0.5)
     n = _ws_bytes(ops, M, K, N, G)
-    assert n > 0
+    assert n > 0 and ops.lib().lhq_selftest_w4_stream(M, N, K, G, 1) == 0
     ws = torch.empty(n, dtype=torch.uint8, device="cuda")
     C = ops.dev(C0)
     C0d = ops.dev(C0)

@@ -51,8 +51,8 @@ def _case(oracle, ops, M, K, N, G, seed):
     (4, 16384, 8192, 128),    # 4 rows, K >= 16384
     (17, 4096, 8200, 128),    # 32-row blocks, N % 16 != 0
     (32, 2048, 16400, 256),   # G = 256: two K tiles per scale group
-    (48, 2048, 1024, 128),    # 64-row blocks, 48 live rows
-    (56, 1152, 2048, 384),    # G = 384: split boundary inside a scale group
+    (48, 4096, 1024, 128),    # 64-row blocks, 48 live rows
+    (56, 2304, 2048, 384),    # G = 384: split boundary inside a scale group
     (64, 8192, 1024, 128),    # config 5 K
     (64, 4096, 4104, 128),    # ragged N at 64 rows
     (24, 16384, 2064, 128),   # K >= 16384: 32-row blocks, K halves in the workgroup, odd K tiles per split
@@ -65,6 +65,7 @@ def test_splitk_matches_oracle(oracle, ops, M, K, N, G):
     A, w, want = _case(oracle, ops, M, K, N, G, seed=700 + M + N)
     need = ops.lib().lhq_gemm_w4a16_bf16_workspace_bytes(M, N, K, G)
     assert need > 0 and need % (M * N * 4) == 0, need
+    assert ops.lib().lhq_selftest_w4_stream(M, N, K, G, 0) == 0  # the kernel that needs no split leaves it
     ws = ops.w4a16_bf16_workspace(M, w)
     print(f"split-K M={M} K={K} N={N} G={G}: {need // (M * N * 4)} splits", flush=True)
     got = D.bf16_bits_to_f32(ops.host(ops.gemm_w4a16_bf16_ws(A, w, ws), np.uint16))
@@ -76,7 +77,9 @@ def test_splitk_deterministic_and_workspace_rules(oracle, ops):
     """Same inputs, same workspace size: identical bits on every call.  A
     workspace smaller than asked runs fewer splits and one of none runs
     unsplit; both stay within the bars."""
-    for M, K, N, G in ((24, 4096, 8192, 128), (64, 8192, 2048, 128)):
+    for M, K, N, G in ((24, 4096, 8200, 128), (64, 8192, 2048, 128)):
+        assert ops.lib().lhq_selftest_w4_stream(M, N, K, G, 0) == 0
+        assert ops.lib().lhq_gemm_w4a16_bf16_workspace_bytes(M, N, K, G) > 2 * M * N * 4
         _deterministic(oracle, ops, M, K, N, G)
 
 

@@ -33,11 +33,11 @@ def _case(oracle, ops, M, K, N, seed):
 def test_noalloc_matches_workspace_entry_on_consecutive_calls(oracle, ops):
     # the second call is smaller (fewer rows, shorter K, less scratch), and
     # both split K
-    for M, K, N in ((64, 8192, 8192), (24, 4096, 8192)):
+    for M, K, N in ((64, 8192, 8192), (24, 4096, 8200)):
         A, w, want = _case(oracle, ops, M, K, N, seed=M + N)
         need = ops.lib().lhq_gemm_w4a16_bf16_workspace_bytes(M, N, K, 128)
         print(f"noalloc M={M} K={K} N={N}: {need} bytes of scratch", flush=True)
-        assert need > 0
+        assert need > 0 and ops.lib().lhq_selftest_w4_stream(M, N, K, 128, 0) == 0
         ref = ops.host(ops.gemm_w4a16_bf16_ws(A, w, ops.w4a16_bf16_workspace(M, w)), np.uint16)
         got = ops.host(ops.gemm_w4a16_bf16_noalloc(A, w, ops.empty((M, N), np.int16)), np.uint16)
         assert np.array_equal(got, ref)

@@ -393,6 +393,11 @@ int lhq_selftest_bf16(unsigned long long* counts, void* stream);
  * f32 != 0: lhq_gemm_w4a16 and _ws.  For tests, which assert the kernel they
  * mean to run. */
 int lhq_selftest_w4_stream(int M, int N, int K, int G, int f32);
+/* The same for the 8-bit GEMMs (fp8 = 0: lhq_gemm_w8a8, _bf16 and _i32): 16 *
+ * (16-row blocks) + column tiles per workgroup, + 256 with a window of 8 loads
+ * instead of 16, + 512 where the activations go through on-chip memory in
+ * phases; 0 where another kernel takes the call. */
+int lhq_selftest_gemm8_stream(int M, int N, int K, int fp8);
 /* The matrix-core rate probes bench.py uses are in the separate diagnostics
  * library (include/longhorn_diag.h, liblonghorn_diag.so). */
 

@@ -21,8 +21,9 @@
 // its L2 sees the A rows and B columns they share.  Where the tiles fill at
 // most half the CUs, every workgroup takes a 256x128 half tile instead; up to
 // 64 rows gemm8_stream_kernel stages A in LDS and streams B past it (the
-// M = 1 GEMV and batched decode; where A's rows are not 16-byte aligned,
-// gemm8_mid_kernel reads both straight from global memory up to 32 rows).
+// M = 1 GEMV and batched decode; where stream_wins says so or A's rows are
+// not 16-byte aligned, gemm8_mid_kernel reads both straight from global
+// memory up to 32 rows and the half tiles take more).
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -1136,11 +1137,12 @@ __device__ __forceinline__ void store_block16(const Gemm8Args& p, const Acc& acc
 }
 
 // ---------------------------------------------------------------------------
-// Small- and mid-size int8 kernel (W8A8 with M <= kMidMaxM: the M = 1 GEMV
-// of config 1 and batched decode).  There the 256x256 tile kernel runs
-// ceil(N/256) workgroups -- 56 at N = 14336, under a quarter of the CUs --
-// each walking all of K, and the rows past M are MFMA work for nothing.  Here a 64 W-thread workgroup owns an
-// output block of RB 16-row blocks by T 16-column tiles and its W waves
+// Small- and mid-size kernel (M <= kMidMaxM where gemm8_stream_kernel below
+// does not take the call: M up to 12 at some K and N, any where A is not
+// 16-byte aligned).  There the 256x256 tile kernel runs ceil(N/256)
+// workgroups -- 56 at N = 14336, under a quarter of the CUs -- each walking
+// all of K, and the rows past M are MFMA work for nothing.  Here a 64 W-thread
+// workgroup owns an output block of RB 16-row blocks by T 16-column tiles and its W waves
 // split K; per 64-deep k step a lane loads 16 contiguous k bytes of each of
 // its T B^T columns and RB A rows (1 KiB loads per wave), and RB * T
 // v_mfma_i32_16x16x64_i8 accumulate the blocks (rows past M read row M-1,
@@ -1255,11 +1257,12 @@ __global__ __launch_bounds__(64 * W, MINW) void gemm8_mid_kernel(Gemm8Args p) {
 // are neither staged nor stored (their LDS words reach only their own D
 // rows).  The K parts' blocks meet in LDS in K order, the epilogue is the
 // kernel's above: int32 sums exactly, fp32 ones in a fixed order.
-// Measured (us a call, int8; before = the kernel above up to 32 rows, 256 x
-// 128 half tiles from 33): K = 4096, N = 14336 M = 1 14.3 -> 13.5, 16 18.8 ->
-// 14.7, 24 22.0 -> 15.6, 32 23.7 -> 16.0, 64 31.2 -> 19.8; K = N = 4096 M = 32
-// 13.6 -> 8.7, 64 28.6 -> 14.4; K = N = 8192 M = 1 15.8 -> 16.2, 16 19.8 ->
-// 18.9, 64 52.7 -> 25.1.  The weights' read bounds it (4.4 TB/s at M = 1).
+// Measured (us a call, int8; the kernel above up to 32 rows and 256 x 128
+// half tiles from 33 / this one): K = 4096, N = 14336 M = 1 14.2 / 13.7, 16
+// 18.4 / 14.2, 24 21.4 / 15.3, 32 22.9 / 15.5, 64 29.7 / 19.1; K = N = 4096 M =
+// 32 11.8 / 7.7, 64 23.7 / 14.2; K = N = 8192 M = 1 15.9 / 14.6, 16 19.5 / 16.4,
+// 64 51.8 / 25.6.  The weights' read bounds it (4.3 TB/s at M = 1).  Where the
+// others win (some few rows and two rounds of the CUs): stream_wins.
 // ---------------------------------------------------------------------------
 constexpr int kStreamWindow = 16;
 constexpr int stream_waves(int CT) { return CT == 3 ? 6 : 8; }
@@ -1406,6 +1409,7 @@ int device_cus() {
 constexpr size_t kStreamLds = 144 * 1024;  // A's buffers
 struct StreamPlan {
     int ct = 0, sp = 0, phases = 0, pitch = 0;
+    int64_t rounds = 0;  // of the CUs
     size_t lds = 0;
 };
 StreamPlan plan_stream(const Gemm8Args& p, int rb) {
@@ -1432,16 +1436,59 @@ StreamPlan plan_stream(const Gemm8Args& p, int rb) {
         }
         const size_t a = static_cast<size_t>(t.phases > 1 ? 2 : 1) * 16 * rb * t.pitch;
         t.lds = std::max(a, static_cast<size_t>(kp - 1) * ct * rb * 1024);
-        // rounds of the CUs times the tiles of a workgroup; ties to the wider
-        // one, which stages A less often
-        const int64_t wgs = ceil_div(nt, ct);
-        const int64_t cost = ceil_div64(wgs, static_cast<int64_t>(cus)) * ct;
+        // rounds of the CUs, a round being a workgroup's tiles and the staging
+        // of A with the K parts' meeting (about half a tile's time); ties to
+        // the wider one, which stages A less often
+        t.rounds = ceil_div64(ceil_div(nt, ct), static_cast<int64_t>(cus));
+        const int64_t cost = t.rounds * (2 * ct + 1);
         if (best.ct == 0 || cost < best_cost) {
             best = t;
             best_cost = cost;
         }
     }
     return best;
+}
+
+// Where the kernels beside it are the faster ones, from some 4,600 shapes
+// timed with both, of either type (us, those / this, int8):
+//   M > 32 (256 x 128 half tiles there) once the tiles take two rounds of the
+//     CUs: staging 64 rows by every workgroup costs what K is too short to
+//     repay, above all where one workgroup fills a CU's LDS (K past 1280).
+//     M=64, N=20480: K=512 8.0 / 9.6, K=1024 11.2 / 10.2, K=1408 13.9 / 18.9,
+//     K=2048 17.9 / 20.3, K=3072 25.8 / 26.0, K=4096 31.5 / 31.5; M=33, K=1408
+//     13.5 / 15.2; one round: M=64, K=256, N=14336 6.6 / 7.6
+//   M <= 12 (16-row blocks straight from memory there), K a multiple of 4096:
+//     with few K parts per workgroup the rows of B^T, that far apart, meet in
+//     few memory channels: K=8192, N=17920 M=1 31.0 / 38.1, M=8 35.3 / 39.3,
+//     M=12 38.4 / 39.7; K=12288, N=18432 M=4 49.4 / 53.4; K=4096, N=8192 M=8
+//     9.9 / 10.4; but K=8192, N=14336 M=4 27.0 / 25.3, K=9216, N=18432 M=2
+//     44.3 / 40.9
+//   M <= 2, a second round that is a quarter full: K=4096, N=17920 M=1 16.6 /
+//     17.9; but K=5120 29.4 / 24.6
+template <int OP>
+bool stream_wins(const Gemm8Args& p, const StreamPlan& t) {
+    const int M = p.M, K = p.Kp, nt = ceil_div(p.N, 16), cus = std::max(device_cus(), 1);
+    constexpr bool I8 = OP == OP_I8;
+    if (M > 32) {
+        if (t.rounds == 1) return !(I8 && M > 33 && K <= 384 && nt > (M > 48 ? 5 * cus / 2 : 3 * cus));
+        if (K <= 2304) {
+            const int shortest = I8 ? (M < 40 ? 512 : M <= 48 ? 640 : 896) : M <= 40 ? 512 : 640;
+            return !(K <= shortest || (K > 1024 && K != 1280) || (K == 1280 && I8 && M > 56));
+        }
+        return !(M >= 40 && K <= 4096 && (nt > 6 * cus || (M > 48 && (K <= 2560 || (K > 3072 && K <= 3584)))));
+    }
+    if (M > 12) return true;
+    if (K == 8192 && ((M <= (I8 ? 12 : 10) && nt >= 4 * cus) ||
+                      (M <= 4 && 2 * nt > 5 * cus && nt <= 3 * cus) ||
+                      (M <= 8 && 8 * nt > 23 * cus && nt <= 3 * cus) ||
+                      (M == 1 && 2 * nt > 5 * cus)))
+        return false;
+    if (K == 12288 && M <= 4 && nt > 4 * cus) return false;
+    if (K == 4096 && M <= 8 && 4 * nt > 7 * cus && nt <= 2 * cus) return false;
+    if (M <= 2 && nt > 4 * cus && nt <= 5 * cus &&
+        ((M == 1 && K > 2048 && K <= 4096) || (K > 6144 && K <= 8192) || K > 9216))
+        return false;
+    return !(M == 1 && nt > 6 * cus && (K == 4096 || K == 14336));
 }
 
 template <int EPI, int RB, int CT, int OP, int D>
@@ -1548,15 +1595,19 @@ int launch_gemm8(const uint8_t* A, const uint8_t* Bt, const float* As, const flo
     // of A before it reaches the MFMA
     static const int use_dma = env_int("LHQ_GEMM8_DMA", 1);
     static const int use_small = env_int("LHQ_GEMM8_SKINNY", 1);
-    // up to 64 rows: A staged in LDS, one pass over the weights (its loads
-    // need 16-byte aligned rows; from 65 rows a second pass costs what the
-    // half tiles do: K = N = 8192 M = 64 25 us, M = 65 on half tiles 53)
+    // up to 64 rows: A staged in LDS, one pass over the weights, where that
+    // wins (its loads need 16-byte aligned rows; from 65 rows a second pass
+    // costs what the half tiles do: K = N = 8192 M = 64 25 us, M = 65 on half
+    // tiles 53)
     static const int env_stream = env_int("LHQ_GEMM8_STREAM", 64);
     if (M <= env_stream && (OP == OP_I8 || K % BK == 0) && (reinterpret_cast<uintptr_t>(A) & 15) == 0) {
         const StreamPlan t = plan_stream(p, M <= 16 ? 1 : M <= 32 ? 2 : 4);
-        if (t.ct && M <= 16) return launch_stream<EPI, 1, OP>(p, t, stream, who);
-        if (t.ct && M <= 32) return launch_stream<EPI, 2, OP>(p, t, stream, who);
-        if (t.ct) return launch_stream<EPI, 4, OP>(p, t, stream, who);
+        static const bool always = env_int("LHQ_GEMM8_STREAM", 0) > 0;
+        if (t.ct && (always || stream_wins<OP>(p, t))) {
+            if (M <= 16) return launch_stream<EPI, 1, OP>(p, t, stream, who);
+            if (M <= 32) return launch_stream<EPI, 2, OP>(p, t, stream, who);
+            return launch_stream<EPI, 4, OP>(p, t, stream, who);
+        }
     }
     if constexpr (OP == OP_FP8) {
         // up to 32 rows (K % 128 == 0): the mid-size kernel's 32 x 32 blocks.
@@ -1673,6 +1724,19 @@ int lhq_gemm_fp8_e4m3(const uint8_t* A, const uint8_t* Bt, const float* A_scale,
                       float* C, int M, int N, int K, float alpha, float beta, void* stream) {
     return launch_gemm8<OP_FP8, EPI_F32>(A, Bt, A_scale, B_scale, C, M, N, K, alpha, beta, stream,
                                          "gemm_fp8_e4m3");
+}
+
+int lhq_selftest_gemm8_stream(int M, int N, int K, int fp8) {
+    if (M <= 0 || N <= 0 || K <= 0 || M > 64 || (fp8 && K % BK != 0) || K % 16 != 0) return 0;
+    Gemm8Args p{};
+    p.M = M;
+    p.N = N;
+    p.K = K;
+    p.Kp = ceil_div(K, BK) * BK;
+    const int rb = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    const StreamPlan t = plan_stream(p, rb);
+    if (!t.ct || !(fp8 ? stream_wins<OP_FP8>(p, t) : stream_wins<OP_I8>(p, t))) return 0;
+    return 16 * rb + t.ct + (t.sp <= 8 ? 256 : 0) + (t.phases > 1 ? 512 : 0);
 }
 
 }  // extern "C"

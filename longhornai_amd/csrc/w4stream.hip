@@ -1,5 +1,7 @@
-// w4stream.hip -- W4A16 for a few rows of a plain call: 5..64 in bf16, 5..32
-// of the fp32 interface, where w4_stream_rb finds it the fastest.
+// w4stream.hip -- W4A16 for a few rows: 5..64 in bf16 (the workspace and the
+// no-allocation entry points; lhq_gemm_w4a16_bf16 and the batched and grouped
+// ones keep the kernels beside it), 5..32 of the fp32 interface, where
+// w4_stream_rb finds it the fastest.
 //
 // The weights' read bounds these calls (K=8192, N=28672 at G=32: 132 MB, 20 us
 // at 6.5 TB/s), and below about 20 MB of weights the launch.  The kernels
@@ -325,6 +327,89 @@ int column_tiles(const W4Args& a, bool f32, int rb, int cus) {
     return ct;
 }
 
+// Where this kernel is the fastest, from 36,839 shapes timed with it and with
+// the kernels beside it (those / this, us): with this rule the mean over all
+// of them is 0.93 / 0.88 / 0.84 of theirs (G = 128, 64, 32; fp32 0.84), and about
+// one in a thousand is 2 to 5% slower.  Every workgroup stages the rows, about two column tiles' time,
+// growing with M K; a round of the CUs that is barely begun is lost; and the
+// 16-row kernel, which gives a workgroup one column tile and two waves' worth
+// of K each, is at its best where the tiles just fill a round of two (or, up
+// to 14 rows, one) per CU.
+bool stream_wins(const W4Args& a, bool f32, int ct) {
+    const int M = a.M, K = a.K, G = a.G, cus = std::max(w4_device_cus(), 1);
+    const int rounds = ceil_div(ceil_div(a.Nt, ct), cus);
+    const int u = static_cast<int>(ceil_div64(int64_t{a.Nt} * 64, cus));  // 64ths of a column tile per CU
+    const bool one = rounds == 1, full = 4 * int64_t{a.Nt} >= int64_t{3} * rounds * ct * cus;
+    const bool fine = G < kW4TileK;          // several scale groups per K tile
+    const bool brief = K > 512 && K < 1024;  // five to seven K tiles over eight waves
+    if (f32) {  // twice the bytes to stage, and coarse groups only
+        // M=17, N=12288: K=2048 13.8 / 11.7; N=1024, M=32, K=768 5.5 / 5.9
+        if (M > 16) return (one && K <= 1024 && (K == 1024 || u > 32)) || (u <= 192 && K > 1024 && K <= 2048);
+        // M=16: K=2048, N=14336 14.4 / 9.2; K=4096, N=8192 13.1 / 10.9; K=14336, N=512 38.9 / 21.2
+        if ((M == 5 || M == 9) && K > 1024 && K < 1280) return false;
+        if (M > 8) return (one && K <= 2048) || (u <= 128 && K <= 4096) || u <= 32;
+        // M=5, N=4096: K=768 4.0 / 4.1, K=2304 5.4 / 5.9, K=4096 7.3 / 7.4, K=5632 16.3 / 9.4
+        if (ct == 1 && ((K > 1024 && K <= 2304) || (M == 5 ? K < 5120 : M <= 7 && K > 3072 && K < (M == 6 ? 4480 : 4096))))
+            return false;
+        if (ct == 4 && M <= 7 && K < 1024) return false;
+        return (one && K <= 4096) || (u <= 64 && K <= 8192) || u <= 32;
+    }
+    if (M <= 8) {
+        // four tiles each: M=8, N=14336: K=4096 14.5 / 10.6, but K=5120 12.2 / 13.3
+        if (ct != 4 || !full) return false;
+        if (!one)
+            return !fine     ? K >= 8192  // N=28672: M=8 31.6 / 31.1
+                   : G == 64 ? K > 5632 || (u > 384 && K > 2048 && K <= 4096)
+                             : K > 2048;
+        if (!fine) return K > 2560 && u > 200 && K <= (M <= 6 ? 5120 : 4096) && (M > 6 || u <= 240);
+        if (M <= 6) return K > (G == 64 ? 2048 : 3072) && (u > 200 || K > 5120);
+        return K > 2048 && (u > 200 || K > 3072);
+    }
+    if (M <= 16) {
+        if (!one) return full && K > 1024 && K <= 2048;  // N=28672, M=16: K=2048 16.5 / 11.2, K=4096 20.6 / 21.0
+        if (brief && M <= 10 && ct != 2 && u <= 192) return false;
+        if (ct == 2) {
+            // M=13, K=7168: N=7168 14.7 / 11.6, but with the round full N=8192 11.1 / 12.2
+            if (u > 124 && K > 2048) return false;
+            if (!fine) return !(M <= 10 && K > 4096 && K <= 4864 && u > 100);
+            return M > (G == 64 ? 10 : 12) || (K >= 1024 && !(G == 64 && K > 4096 && K <= 4608));
+        }
+        if (ct == 4) {
+            // M=16, N=12288: K=2560 9.4 / 8.7 (M=13 slower), K=4096 12.9 / 10.7, K=14336 24.6 / 28.0
+            if (!fine) return K <= 2048 || (full && (M <= 10 ? K <= 4096 : (K > 3072 && K <= 4096) || (M <= 14 && K <= 2304)));
+            return G == 64 ? M > 10 || !brief : M > 12 ? !brief : K >= 1536;
+        }
+        // one tile each: M=9, N=4096: K=2048 4.8 / 4.7, K=5632 6.1 / 6.9; M=16: any
+        if (!fine) {
+            if (M <= 10) return (K <= 4096 && !(K > 1536 && K < 2048)) || u <= 16;
+            if (M <= 14 && K > 4096 && K < 4608) return false;
+            return M > 14 || u <= (M <= 12 ? 40 : 16) || !(K > (M <= 12 ? 4096 : 3584) && K <= 5632);
+        }
+        if (G == 64) {
+            if (M <= 10) return K > 2304 && K <= 4608;
+            return M > 14 || !(K > (M <= 12 ? 4096 : 3072) && K <= 5632);
+        }
+        if (M <= 12) return (K > 2304 && K <= 3584) || K > 5632;
+        return !brief && !(K > 3584 && K <= 4608) && (M > 14 || !((K > 1024 && K < 1536) || (K > 1792 && K <= 2304)));
+    }
+    // under 1.5 tiles per CU the 16-row kernel wins to 47 rows (K=N=4096, M=32
+    // 7.4 / 8.4; M=33, K=1024, N=2048 3.6 / 5.5), this one from 48 (K=2048, N=3072
+    // 12.3 / 7.9)
+    if (u < 96) return M >= 48 && one && K <= 2048 && !fine;
+    if (M <= 32) {
+        if (fine) return (one || full) && (K >= 768 || u > 124);  // G=32, M=24, K=4096, N=28672 40.6 / 30.4
+        // M=17, N=7168: K=512 4.1 / 4.4, K=1536 6.4 / 6.1, K=2304 7.0 / 7.4
+        if (u <= 124) return K >= 1024 && K <= 4096 && !(M <= 24 && K > 1792 && K <= 2304);
+        // M=32: K=2048, N=16384 14.2 / 10.1; N=8192: K=4096 14.4 / 11.1, K=8192 16.8 / 18.3
+        return (one && K <= 2048) || (rounds == 2 && K >= 512 && K <= 1024) || (u <= 128 && K <= 4096);
+    }
+    // a second pair of tiles for a few CUs only: M=48, G=64, K=8192: N=10240 34.2 / 41.0, N=11008 49.5 / 41.4
+    const bool gap = u > 128 && u <= 170;
+    if (fine) return (one || (full && !(G == 64 && K >= 8192))) && !(G == 64 && M < 64 && K >= 2048 && gap);
+    // M=64, N=14336: K=2048 19.6 / 12.9, K=4096 20.8 / 22.0, K=8192 31.8 / 39.1
+    return (one && K <= 2048 && !(M < 48 && K > 1536 && gap)) || (u <= 128 && K <= 4096);
+}
+
 }  // namespace
 
 int w4_stream_rb(const W4Args& a, bool f32) {
@@ -334,52 +419,8 @@ int w4_stream_rb(const W4Args& a, bool f32) {
         (reinterpret_cast<uintptr_t>(a.A) & 15) != 0 || static_cast<int64_t>(M) * K * (f32 ? 4 : 2) >= (int64_t{1} << 31))
         return 0;
     const int env = tuning_knob("LHQ_W4S", -1);  // 0: never; 1: always
-    // Where the lines lie (us on the other kernels / on this one).  The staging
-    // costs a round of the CUs about two tiles and grows with M K, so: fine
-    // scale groups (G < 128, which the tiles do not take: their 16-row kernel
-    // re-reads the rows) win for every grid that fills its rounds to 3/4 --
-    // N=28672, M=24, K=4096 40.8 / 30.5; N=20480 (62%), M=48 32.9 / 37.4.
-    // From G = 128 on:
-    //   M 5..8    four tiles each and long K: N=28672 K=8192 34.0 / 30.4, but
-    //             two tiles (N=8192, K=8192) 10.2 / 11.6, K=7168 N=15360 16.1 / 16.7
-    //   M 9..16   N <= 8192 at any K (8192 x 8192: 13.1 / 12.6), else one round and
-    //             K <= 4096 (K=14336, N=12288 24.8 / 28.2); two rounds K in
-    //             (1024, 2048] (N=28672: K=2048 16.2 / 10.7, K=4096 20.1 / 21.0)
-    //   M 17..32  K <= 2048 (N=16384 11.9 / 10.4), or N <= 8192 and K <= 4096 (12.1 /
-    //             11.5; K=8192 16.0 / 17.8); under 1.5 tiles per CU both wait for
-    //             the launch, or the 16-row kernel wins (K=N=4096 7.7 / 8.6)
-    //   M 33..64  the same (K=2048, N=14336 15.8 / 13.8, K=4096 20.5 / 20.3, K=8192
-    //             33.2 / 37.6); under 1.5 tiles the 16-row kernel keeps M < 48 past
-    //             K = 1024 (K=2048, N=3000, M=33 6.8 / 7.7, M=56 12.2 / 8.4)
-    // fp32 (twice the bytes to stage, G >= 128 only):
-    //   M 5..8    one round and K <= 4096 (N=14336 14.1 / 13.6); N <= 4096 to K = 8192
-    //             (14.4 / 13.5); N <= 2048 always (K=14336 36.2 / 18.8)
-    //   M 9..16   one round and K <= 2048 (N=14336 14.3 / 9.8); N <= 8192 to K = 4096
-    //             (12.1 / 11.7; K=8192 17.7 / 18.7); N <= 2048 always (38.5 / 22.2)
-    //   M 17..32  one round and K <= 1024 (N=16384 13.2 / 9.3); N <= 12288 to K = 2048
-    //             (14.0 / 13.9; K=4096 19.0 / 21.8)
     if (env == 0 || env == 1) return env ? rb : 0;
-    const int cus = std::max(w4_device_cus(), 1), Nt = a.Nt, ct = column_tiles(a, f32, rb, cus);
-    const int rounds = ceil_div(ceil_div(Nt, ct), cus);
-    const bool one = rounds == 1, wide = 2 * Nt >= 3 * cus, segs = a.G < kW4TileK;
-    const bool full = 4 * int64_t{Nt} >= int64_t{3} * rounds * ct * cus, two = rounds == 2 && full;
-    bool take;
-    if (f32) {
-        take = M > 16  ? (one && K <= 1024) || (Nt <= 3 * cus && K <= 2048)
-               : M > 8 ? (one && K <= 2048) || (Nt <= 2 * cus && K <= 4096) || 2 * Nt <= cus
-                       : (one && K <= 4096) || (Nt <= cus && K <= 8192) || 2 * Nt <= cus;
-    } else if (M <= 8) {
-        take = ct == 4 && K > 2048 && full && (one ? segs || K <= 5120 : two && (segs || K >= 8192));
-    } else if (M <= 16) {
-        take = one ? segs || Nt <= 2 * cus || K <= 2048 || (full && K <= 4096) : two && K > 1024 && K <= 2048;
-    } else if (segs) {
-        take = wide && (one || full);
-    } else if (M <= 32) {
-        take = wide && ((one && K <= 2048) || (rounds == 2 && K >= 512 && K <= 1024) || (Nt <= 2 * cus && K <= 4096));
-    } else {
-        take = (one && K <= 2048 && (wide || M >= 48 || K <= 1024)) || (wide && Nt <= 2 * cus && K <= 4096);
-    }
-    return take ? rb : 0;
+    return stream_wins(a, f32, column_tiles(a, f32, rb, std::max(w4_device_cus(), 1))) ? rb : 0;
 }
 
 int launch_w4_stream(const W4Args& a, bool f32, int rb, hipStream_t s, const char* who) {

@@ -2772,25 +2772,30 @@ W4Args grouped_args(const uint16_t* A, const int32_t* offsets, const uint8_t* co
     a.row_capacity = row_capacity;
     return a;
 }
-// Tiles for a grouped launch with a workspace.  The persistent launch shares its tiles out
-// over the CUs, so with a 256-column tile per CU or more among all groups'
-// columns (or long K behind fewer) it wins from about 12 rows per group on,
-// where every group still wastes most of its 64-row tile: the 16-row kernel
-// reads the rows from L2 for every column tile, and the weights again for
-// each 16 of them.  us of a MoE layer, that launch on the 16-row kernel / on
-// tiles, at 16 and 40 rows per group:
-//   64 experts, gate / up K=4096, 2 x 1792 columns: 299 / 267, 486 / 376;
-//               down K=1792, 4096 columns: 299 / 283, 486 / 434
-//   8 experts,  gate / up K=2048, 2 x 5632: 71 / 69, 114 / 86;
-//               down K=14336, 4096 (128 tiles): 274 / 269, 449 / 408
-//   but 8 experts of K=1024, 2 x 2048 (128 tiles) 37 / 41, 48 / 52, and
-//   down K=5632, 2048 (64 tiles) 71 / 77, 114 / 114
+// Tiles for a grouped launch with a workspace, from 16 rows per group on.  The
+// persistent launch shares its tiles out over the CUs; the 16-row kernel reads
+// the rows from L2 for every column tile, and the weights again for each 16 of
+// them.  Up to some 36 rows, where every group still wastes much of its 64-row
+// tile, it takes a quarter more 256-column tiles than CUs among all groups'
+// columns, or long K to spread over idle CUs.  us of one launch on the 16-row
+// kernel / on tiles (3,402 shapes of 8, 16 and 64 groups measured):
+//   16 rows: K=1024, 288 tiles 21.4 / 33.1, 384 26.3 / 22.2; K=4096, 1024 tiles
+//            196 / 161; K=14336, 128 tiles 100 / 78
+//   18 rows: K=2560, 256 tiles 34.7 / 44.3, 320 50.8 / 42.1; K=8192, 224 tiles 77.7 / 84.1
+//   24 rows: K=1024, 256 tiles 21.7 / 27.2; K=8192, 192 tiles 82 / 70
+//   32 rows: K=1024, 256 tiles 25.5 / 33.1; K=1792 41.5 / 41.6
+//   40 rows: K=1024, 128 tiles 19.2 / 21.5, 256 29.1 / 21.8; K=4096, 1024 tiles 344 / 215
 bool grouped_uses_tiles(const W4Args& a) {
     const double rows = static_cast<double>(a.row_capacity) / a.num_groups;
     if (mma_applies(a, a.row_capacity, rows)) return true;
-    const int64_t tiles = static_cast<int64_t>(a.num_groups) * a.Nt / 16;
-    return mma_takes(a, a.row_capacity) && rows >= 16.0 &&
-           (tiles >= device_cus() || tiles * a.K >= (int64_t{3} << 19));
+    if (!mma_takes(a, a.row_capacity) || rows < 16.0) return false;
+    const int64_t tiles = static_cast<int64_t>(a.num_groups) * a.Nt / 16, cus = device_cus();
+    const bool deep = tiles * a.K >= (int64_t{3} << 19);
+    if (rows >= 36.0) return tiles >= cus || deep;
+    if (rows >= 28.0) return 4 * tiles >= 5 * cus || (tiles >= cus && a.K >= 1792) || deep;
+    if (4 * tiles >= 5 * cus) return 2 * tiles >= 3 * cus || (rows >= 18.0 && a.K >= 1792);
+    if (tiles >= cus) return a.K >= 4096 && a.K <= (rows >= 20.0 ? 8192 : 5632);
+    return deep && (rows >= 20.0 || 2 * tiles <= cus);
 }
 
 // Partial-sum slots a persistent grouped launch can use: a split of R = T

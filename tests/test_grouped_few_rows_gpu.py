@@ -17,12 +17,17 @@ def ops(lib):
 
 
 @pytest.mark.parametrize("rows,K,N,G,swiglu,tiles", [
-    ([16] * 16, 512, 4096, 128, False, True),            # 256 column tiles, exactly 16 rows
-    ([15] * 15 + [30], 512, 4096, 128, False, False),    # 15.9
-    ([0, 1, 97, 16, 3, 65, 5, 12] * 2, 256, 4100, 256, False, True),
+    ([16] * 16, 512, 6144, 128, False, True),            # 384 column tiles, exactly 16 rows
+    ([15] * 15 + [30], 512, 6144, 128, False, False),    # 15.9
+    ([16] * 16, 512, 4096, 128, False, False),           # 256 column tiles
+    ([0, 1, 97, 16, 3, 65, 5, 12] * 2, 256, 6200, 256, False, True),
+    ([18] * 16, 1792, 5120, 128, False, True),           # 320
+    ([17] * 16, 1792, 5120, 128, False, False),
+    ([35] * 16, 512, 4096, 128, False, False),           # 256, and the row line that takes them
+    ([36] * 16, 512, 4096, 128, False, True),
     ([40] * 15, 512, 4096, 128, False, False),           # 240 column tiles, short K
     ([17, 40] * 4, 12288, 4096, 128, False, True),       # 128, long K
-    ([33] * 8, 512, 4096, 128, True, True),              # gate and up: 512
+    ([33] * 8, 512, 6144, 128, True, True),              # gate and up: 384
     ([20, 40, 10], 384, 1000, 128, True, False),
 ])
 def test_both_sides(oracle, ops, rows, K, N, G, swiglu, tiles):
@@ -35,8 +40,9 @@ def test_both_sides(oracle, ops, rows, K, N, G, swiglu, tiles):
 
 
 def test_workspaces_it_does_not_use(oracle, ops):
-    c = Case(oracle, ops, [20] * 16, 256, 4096, 128, seed=4)
+    c = Case(oracle, ops, [20] * 16, 256, 6144, 128, seed=4)
     need = c.workspace_bytes(ops)
+    assert need > 0
     plain = c.run(ops)
     c.check(oracle, plain)
     assert (c.run(ops, _workspace(ops, need), SLOT - 16) == plain).all()

@@ -14,8 +14,8 @@
 // took 265 us.)  The partial tiles meet in LDS in wave order, so results are
 // deterministic; many short sums instead of one long one also halve the
 // error.  K = N = 4096: M = 100 51 us, 66 TFLOP/s (the 64x64 VALU tile that
-// walked all of K took 550); M = 1 28 us, 2.4 TB/s of B (502); M = 512 175 us,
-// 98 TFLOP/s (584).
+// walks all of K 550); M = 1 28 us, 2.4 TB/s of B (502); M = 512 175 us, 98
+// TFLOP/s (584).  Short K on many outputs stays on that tile (valu_wins).
 //
 // Semantics follow gemm.cpp: lh::gemm applies beta first and never reads C
 // when beta == 0 (gemm.cpp:60-68); lh::gemm_ref always reads C and returns
@@ -44,11 +44,13 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_kernel(const float* __restri
     B += z * K * static_cast<int64_t>(N);
     C += z * M * static_cast<int64_t>(N);
     // workgroups are dealt to the XCDs round-robin: the row tiles of one
-    // column strip go to one XCD, whose L2 then reads the strip's B once
-    const int xcd = blockIdx.x % kXcds, id = blockIdx.x / kXcds;
+    // column strip go to one XCD, whose L2 then reads the strip's B once; the
+    // strips past a multiple of eight follow in order
+    const int whole_strips = (N + 32 * NI - 1) / (32 * NI) / kXcds * kXcds;
+    const int turn = static_cast<int>(blockIdx.x) - mt * whole_strips;  // < 0: one of the whole eights
+    const int id = turn < 0 ? static_cast<int>(blockIdx.x) / kXcds : turn;
     const int m0 = (id % mt) * 32 * MI;
-    const int n0 = ((id / mt) * kXcds + xcd) * 32 * NI;
-    if (n0 >= N) return;  // uniform per workgroup
+    const int n0 = (turn < 0 ? (id / mt) * kXcds + static_cast<int>(blockIdx.x) % kXcds : whole_strips + id / mt) * 32 * NI;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l = lane & 31, h = lane >> 5;
     const int stages = (K + kStage - 1) / kStage;
@@ -86,15 +88,31 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_kernel(const float* __restri
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) r.a[i][q] = load_f32x4<full.value>(ap[i][q] + k0, K - k0 - 4 * ac);
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (full.value) {
+                    r.a[i][q] = load_f32x4<true>(ap[i][q] + k0, 4);
+                } else {
+                    // k past the end reads the row's last element and becomes
+                    // zero: loads under a condition would wait for each other
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int k = k0 + 4 * ac + e;
+                        const float v = ap[i][q][min(k, K - 1) - 4 * ac];
+                        r.a[i][q][e] = k < K ? v : 0.0f;
+                    }
+                }
+            }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int k = k0 + 8 * t, left = K - k - 4 * h;  // the lane's live k from here on
+            const int k = k0 + 8 * t;
 #pragma unroll
             for (int j = 0; j < NI; ++j)
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    r.b[j][t][u] = full.value || u < left ? bp[j][static_cast<int64_t>(k + u) * N] : 0.0f;
+                for (int u = 0; u < 4; ++u) {
+                    const int ku = full.value ? k + u : min(k + u, K - 1 - 4 * h);
+                    const float v = bp[j][static_cast<int64_t>(ku) * N];
+                    r.b[j][t][u] = full.value || k + u + 4 * h < K ? v : 0.0f;
+                }
         }
     };
     // the wave's own LDS (its part of red): row r's k 4 c .. + 3 in slot c ^ (r & 7)
@@ -173,9 +191,87 @@ template <bool REF, int MI, int NI, int KS>
 void launch_tile(const float* A, const float* B, float* C, int batch, int M, int N, int K, float alpha, float beta,
                  hipStream_t s) {
     const int mt = ceil_div(M, 32 * MI), nt = ceil_div(N, 32 * NI);
-    const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(mt) * ceil_div(nt, kXcds) * kXcds), 1,
-                    static_cast<unsigned>(batch));
+    const dim3 grid(static_cast<unsigned>(mt) * static_cast<unsigned>(nt), 1, static_cast<unsigned>(batch));
     gemm_f32_kernel<REF, MI, NI, KS><<<grid, 64 * KS, 0, s>>>(A, B, C, M, N, K, mt, alpha, beta);
+}
+
+// Short K on many outputs: a 256-thread workgroup owns a 64x64 tile, each
+// thread a 4x4 block of VALU sums, K staged 16 at a time.  The tiles above pay
+// for eight partial tiles in LDS whatever K is.
+// Where it wins, us (this / those; 8,937 shapes measured): K=16, M=512, N=2048
+// 5.9 / 8.3, but M=64, N=257 5.3 / 3.4; K=48, M=512, N=2048 9.1 / 10.1; K=32,
+// M=128, N=1024 6.8 / 3.1; K=80, M=2000, N=2048 19.9 / 22.8; M=2000, N=8192: K=96
+// 64 / 75, K=192 111 / 115, K=256 142 / 130.
+// Its grid has two dimensions for the outputs, so it also takes those past
+// 2^32 threads of the other's one.
+constexpr int T = 64, TK = 16;
+
+template <bool REF>
+__global__ __launch_bounds__(256) void gemm_f32_valu_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                       float* __restrict__ C, int M, int N, int K, float alpha,
+                                                       float beta) {
+    __shared__ float sa[TK][T + 4];
+    __shared__ float sb[TK][T + 4];
+    const int64_t z = blockIdx.z;
+    A += z * M * static_cast<int64_t>(K);
+    B += z * K * static_cast<int64_t>(N);
+    C += z * M * static_cast<int64_t>(N);
+    const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    float acc[4][4] = {};
+    for (int k0 = 0; k0 < K; k0 += TK) {
+        for (int i = threadIdx.x; i < T * TK; i += 256) {
+            const int r = i / TK, c = i % TK;  // A tile: 64 rows x 16 k
+            const int gm = m0 + r, gk = k0 + c;
+            sa[c][r] = (gm < M && gk < K) ? A[static_cast<int64_t>(gm) * K + gk] : 0.0f;
+            const int kr = i / T, nc = i % T;  // B tile: 16 k x 64 cols
+            const int gk2 = k0 + kr, gn = n0 + nc;
+            sb[kr][nc] = (gk2 < K && gn < N) ? B[static_cast<int64_t>(gk2) * N + gn] : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < TK; ++kk) {
+            float a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = sa[kk][ty * 4 + i];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = sb[kk][tx * 4 + j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = m0 + ty * 4 + i;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int n = n0 + tx * 4 + j;
+            if (n >= N) continue;
+            float* c = C + static_cast<int64_t>(m) * N + n;
+            if (REF) {
+                *c = alpha * acc[i][j] + beta * *c;
+            } else {
+                const float base = (beta == 0.0f) ? 0.0f : (beta == 1.0f) ? *c : *c * beta;
+                *c = base + alpha * acc[i][j];
+            }
+        }
+    }
+}
+
+bool valu_wins(int batch, int M, int N, int K) {
+    if (static_cast<int64_t>(ceil_div(M, 64)) * ceil_div(N, 32) >= int64_t{1} << 24) return true;
+    if (K < 24 && (M == 1 || N == 1)) return true;
+    const int64_t tiles = static_cast<int64_t>(batch) * ceil_div(M, 32) * ceil_div(N, 32);
+    const bool rows = M > 16;
+    if (K < 32) return tiles > (rows && K >= 24 ? 512 : M < 3 ? 255 : 256);
+    if (K < 64) return tiles > (!rows ? 256 : K == 32 ? 880 : 512);
+    if (K < 96) return tiles > 1100;
+    if (!rows && K % 32 != 0) return K < 256 && tiles > 2200;
+    return K < 256 && tiles > (K < 128 && K % 32 != 0 ? 4000 : K < 200 ? 7900 : 14000);
 }
 
 template <bool REF>
@@ -186,6 +282,12 @@ int launch(const float* A, const float* B, float* C, int batch, int M, int N, in
     if (batch == 0 || M == 0 || N == 0) return LHQ_OK;
     LHQ_REQUIRE(C && ((A && B) || K == 0), "%s: null pointer", who);
     hipStream_t s = as_stream(stream);
+    static const int env = tuning_knob("LHQ_F32_VALU", -1);
+    if (env < 0 ? valu_wins(batch, M, N, K) : env != 0) {
+        gemm_f32_valu_kernel<REF><<<dim3(ceil_div(N, T), ceil_div(M, T), batch), 256, 0, s>>>(A, B, C, M, N, K, alpha,
+                                                                                             beta);
+        return check_launch(who);
+    }
     auto tiles = [&](int rows, int cols) {
         return static_cast<int64_t>(batch) * ceil_div(M, rows) * ceil_div(N, cols);
     };

@@ -1,6 +1,7 @@
 """fp32 GEMM tiles at their edges: rows and columns around a tile, K around the
 32-deep stage and below one stage per wave, misaligned operands, each launch
-shape, denormals, Inf and NaN, against numpy in 64 bits.
+shape, the VALU tiles of short K beside them, denormals, Inf and NaN, against
+numpy in 64 bits.
 
 Tolerance: every output is a sum of K rounded products in some order, so its
 error is at most K * 2^-24 * sum |a b| (any order, fp32, unit roundoff 2^-24),
@@ -28,11 +29,15 @@ def _check(got, A, B, C0, alpha, beta):
     assert (np.abs(got - want) <= bound).all()
 
 
-# 64x32 tiles on 4 waves from 1024 tiles, on 8 from 256, 32x32 below
+# 64x32 tiles on 4 waves from 1024 tiles, on 8 from 256, 32x32 below; the last
+# three rows are VALU tiles but for their first shape (K, rows and outputs on
+# both sides of that line)
 @pytest.mark.parametrize("M,K,N", [
     (1, 1, 1), (31, 31, 33), (33, 32, 32), (32, 33, 31), (5, 7, 300), (40, 255, 65), (1, 289, 1000),
     (65, 100, 4097), (128, 96, 4095), (129, 70, 4100),
-    (1024, 67, 2049), (4097, 40, 500),
+    (1024, 260, 2049), (4097, 300, 500), (2049, 257, 1030),
+    (33, 23, 600), (1, 23, 600), (300, 23, 1000), (512, 31, 1025), (512, 63, 1025), (17, 32, 16500),
+    (1090, 95, 1025), (1024, 67, 2049), (4097, 40, 500), (65, 16, 4097), (4, 33, 8192), (4, 33, 8193),
 ])
 @pytest.mark.parametrize("lead", [0, 1])
 def test_shapes(ops, M, K, N, lead):
@@ -45,8 +50,8 @@ def test_shapes(ops, M, K, N, lead):
         _check(ops.host(C).reshape(M, N), A, B, C0, alpha, beta)
 
 
-def test_batched(ops):
-    batch, M, K, N = 300, 33, 65, 34
+@pytest.mark.parametrize("batch,M,K,N", [(300, 33, 65, 34), (60, 33, 65, 34), (60, 65, 257, 290), (9, 65, 257, 8200)])
+def test_batched(ops, batch, M, K, N):
     A, B = D.normal((batch, M, K), 1.0, 1), D.normal((batch, K, N), 1.0, 2)
     C0 = D.normal((batch, M, N), 1.0, 3)
     C = ops.dev(C0)

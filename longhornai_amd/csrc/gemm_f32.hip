@@ -123,12 +123,16 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_kernel(const float* __restri
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 *reinterpret_cast<f32x4_t*>(mine + (32 * i + 8 * q + ar) * kStage + 4 * (ac ^ ar)) = r.a[i][q];
+        // the rows were written by other lanes of this wave: LDS is in order
+        // within a wave, the fences keep the compiler to it
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         f32x4_t a[MI][4];
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int i = 0; i < MI; ++i)
                 a[i][t] = *reinterpret_cast<const f32x4_t*>(mine + (32 * i + l) * kStage + 4 * ((2 * t + h) ^ (l & 7)));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll

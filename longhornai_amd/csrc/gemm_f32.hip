@@ -267,6 +267,7 @@ __global__ __launch_bounds__(256) void gemm_f32_valu_kernel(const float* __restr
 }
 
 bool valu_wins(int batch, int M, int N, int K) {
+    if (ceil_div(M, T) > 65535) return false;  // its grid's second dimension ends there
     if (static_cast<int64_t>(ceil_div(M, 64)) * ceil_div(N, 32) >= int64_t{1} << 24) return true;
     if (K < 24 && (M == 1 || N == 1)) return true;
     const int64_t tiles = static_cast<int64_t>(batch) * ceil_div(M, 32) * ceil_div(N, 32);

@@ -66,6 +66,14 @@ def test_empty_sum_and_unread_output(ops):
     ops.run("lhq_gemm_f32", np.ones((3, 2), np.float32), np.ones((2, 5), np.float32), ops.dev(np.full((3, 5), np.nan, np.float32)), 3, 5, 2, 1.0, 0.0)
 
 
+def test_more_rows_than_the_valu_grid_holds(ops):
+    M = 64 * 65535 + 1
+    A = (np.arange(2 * M, dtype=np.int64) % 1021).astype(np.float32).reshape(M, 2)
+    C = ops.empty((M, 1), np.float32)
+    ops.run("lhq_gemm_f32", A, np.array([[1.0], [2.0]], np.float32), C, M, 1, 2, 1.0, 0.0)
+    assert np.array_equal(ops.host(C)[:, 0], A[:, 0] + 2 * A[:, 1])  # whole numbers: exact
+
+
 def test_denormals_and_non_finite(ops):
     M, K, N = 40, 70, 40
     A, B = np.full((M, K), 1e-30, np.float32), np.full((K, N), 1e-12, np.float32)

@@ -63,7 +63,11 @@ def test_empty_sum_and_unread_output(ops):
     C = ops.dev(np.full((3, 5), np.nan, np.float32))
     ops.run("lhq_gemm_f32", None, None, C, 3, 5, 0, 1.0, 0.0)
     assert (ops.host(C) == 0).all()
-    ops.run("lhq_gemm_f32", np.ones((3, 2), np.float32), np.ones((2, 5), np.float32), ops.dev(np.full((3, 5), np.nan, np.float32)), 3, 5, 2, 1.0, 0.0)
+    # one shape for each tile: VALU, 64 x 32 on 4 and 8 waves, 32 x 32 on 8
+    for M, K, N in ((517, 2, 1), (2048, 96, 1024), (100, 257, 4096), (33, 70, 40)):
+        C = ops.dev(np.full((M, N), np.nan, np.float32))
+        ops.run("lhq_gemm_f32", np.ones((M, K), np.float32), np.ones((K, N), np.float32), C, M, N, K, 1.0, 0.0)
+        assert (ops.host(C) == K).all(), (M, K, N)
 
 
 def test_more_rows_than_the_valu_grid_holds(ops):

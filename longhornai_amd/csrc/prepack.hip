@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void w4_prepack_kernel(const uint8_t* __restri
                                                          const uint8_t* __restrict__ zeros,
                                                          uint32_t* __restrict__ zeros_out, int K, int N, int Nt,
                                                          int Kt, int NG, int64_t qblocks, int64_t sblocks) {
-    const int64_t blk = blockIdx.x;
+    const int64_t blk = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
     if (blk < qblocks) {
         const int kt = static_cast<int>(blk % Kt);
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void w4_prepack_kernel(const uint8_t* __restri
                 w4_quad(r, d[j]);
             }
         };
-        if (n0 + 4 <= N) read(Full{});
+        if (n0 <= N - 4) read(Full{});
         else read(Part{});
         u32x4_t* o = reinterpret_cast<u32x4_t*>(qweight + (static_cast<int64_t>(nt) * Kt + kt) * kW4TileBytes) +
                      16 * kq + 4 * (c4 & 3);
@@ -120,7 +120,10 @@ int launch_w4_prepack(const uint8_t* packed, const S* scales, const uint8_t* zer
     const int64_t qb = static_cast<int64_t>(ceil_div(Nt, 16)) * Kt;
     const int64_t sb = ceil_div64(static_cast<int64_t>(Nt) * NG * 16, 256);
     const int64_t zb = ASYM ? ceil_div64(static_cast<int64_t>(Nt) * ceil_div(NG, 8) * 16, 256) : 0;
-    w4_prepack_kernel<ASYM, S><<<static_cast<unsigned>(qb + sb + zb), 256, 0, s>>>(
+    // a second grid dimension past 2^30 threads; the blocks past the last one end
+    // in the last section's own bounds
+    const int64_t total = qb + sb + zb, gx = total < (1 << 22) ? total : 1 << 22;
+    w4_prepack_kernel<ASYM, S><<<dim3(static_cast<unsigned>(gx), static_cast<unsigned>(ceil_div64(total, gx))), 256, 0, s>>>(
         packed, qweight, scales, scales_out, zeros, zeros_out, K, N, Nt, Kt, NG, qb, sb);
     return check_launch(who);
 }
@@ -141,16 +144,18 @@ __global__ __launch_bounds__(256) void b8_prepack_kernel(const uint8_t* __restri
     const int k0 = blockIdx.x * 128, n0 = blockIdx.y * 128;
     const int c4 = threadIdx.x & 31;
     const int n = n0 + 4 * c4;
+    const int cnt = max(N - n, 0);
+    // words past the last column are read from column N - 4 on
+    const int from = N >= 4 ? min(n, N - 4) : n, shift = 8 * min(n - from, 3);
     auto put = [&](auto full) {
-        const int cnt = max(N - n, 0);
         uint32_t r[4][4];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int k = k0 + 4 * (static_cast<int>(threadIdx.x >> 5) + 8 * u) + i;
-                const uint32_t v = load_u8x4<full.value>(B + static_cast<int64_t>(min(k, K - 1)) * N + n, cnt);
-                r[u][i] = k < K ? v : 0u;
+                const uint32_t v = load_u8x4<full.value>(B + static_cast<int64_t>(min(k, K - 1)) * N + from, cnt);
+                r[u][i] = k < K && cnt > 0 ? v >> shift : 0u;
             }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -165,7 +170,7 @@ __global__ __launch_bounds__(256) void b8_prepack_kernel(const uint8_t* __restri
             tile[4 * c4 + 3][kw] = __builtin_amdgcn_perm(y1, x1, 0x07060302u);
         }
     };
-    if (n + 4 <= N) put(Full{});
+    if (N >= 4) put(Full{});
     else put(Part{});
     __syncthreads();
 #pragma unroll

@@ -99,14 +99,15 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_kernel(const T* __restri
 }
 
 // fp32 rows whose length is a multiple of 4: 16-byte loads and 4-byte
-// stores; rows of up to 8 * 4 * kBlock elements stay in registers between
+// stores; rows of up to R * 4 * kBlock elements stay in registers between
 // the max-abs pass and the quantizing pass (one read of the row), longer
 // rows are read again (from L2).  Same rule as quant_per_row_kernel.
-template <bool FP8>
+// R (16-byte chunks a thread keeps) is the least of 1, 2, 4, 8 that holds a
+// row (int8, 512 rows of 1024 2.6 us, 4096 of 512 5.3; eight for all 3.1, 6.8).
+template <bool FP8, int R>
 __global__ __launch_bounds__(kBlock) void quant_per_row_f32_vec_kernel(const float* __restrict__ src,
                                                                        uint8_t* __restrict__ dst,
                                                                        float* __restrict__ scales, int dim) {
-    constexpr int R = 8;  // float4 chunks a thread keeps
     const int64_t base = static_cast<int64_t>(blockIdx.x) * dim;
     const f32x4_t* s4 = reinterpret_cast<const f32x4_t*>(src + base);
     const int n4 = dim >> 2;
@@ -152,7 +153,8 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_f32_vec_kernel(const flo
 // rows of up to R * 8 * kBlock elements stay in registers between the two
 // passes, longer rows are read again (from L2).  Bound by memory: 2048 rows
 // of 4096 move 25 MB in 7.4 us at best (9.6 with a second read of the row).
-// R (16-byte chunks a thread keeps) is the least of 1, 2, 4 that holds a row.
+// R (16-byte chunks a thread keeps) is the least of 1, 2, 4, 8 that holds a row
+// (16 rows of 14336 5.6 us; four and a second read 6.7).
 template <bool FP8, int R>
 __global__ __launch_bounds__(kBlock) void quant_per_row_bf16_vec_kernel(const uint16_t* __restrict__ src,
                                                                         uint8_t* __restrict__ dst,
@@ -178,7 +180,8 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_bf16_vec_kernel(const ui
             keep[r] = i < n8 ? s4[i] : u32x4_t{0, 0, 0, 0};
         }
 #pragma unroll
-        for (int r = 0; r < R; ++r) scan(keep[r]);
+        for (int r = 0; r < R; ++r)
+            if (threadIdx.x + r * kBlock < n8) scan(keep[r]);  // (idle waves skip it)
     } else {
         for (int i = threadIdx.x; i < n8; i += kBlock) scan(s4[i]);
     }
@@ -767,13 +770,20 @@ int quantize_per_row(const T* src, uint8_t* dst, float* scales, int rows, int di
             if (dim <= 8 * kBlock) quant_per_row_bf16_vec_kernel<FP8, 1><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
             else if (dim <= 16 * kBlock)
                 quant_per_row_bf16_vec_kernel<FP8, 2><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
-            else quant_per_row_bf16_vec_kernel<FP8, 4><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            else if (dim <= 32 * kBlock)
+                quant_per_row_bf16_vec_kernel<FP8, 4><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            else quant_per_row_bf16_vec_kernel<FP8, 8><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
             return check_launch(who);
         }
     } else {
         if (dim % 4 == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0 &&
             (reinterpret_cast<uintptr_t>(dst) & 3) == 0) {
-            quant_per_row_f32_vec_kernel<FP8><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            if (dim <= 4 * kBlock) quant_per_row_f32_vec_kernel<FP8, 1><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            else if (dim <= 8 * kBlock)
+                quant_per_row_f32_vec_kernel<FP8, 2><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            else if (dim <= 16 * kBlock)
+                quant_per_row_f32_vec_kernel<FP8, 4><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
+            else quant_per_row_f32_vec_kernel<FP8, 8><<<rows, kBlock, 0, s>>>(src, dst, scales, dim);
             return check_launch(who);
         }
     }

@@ -114,9 +114,9 @@ def test_per_col(oracle, ops, rows, cols, kind):
     _same(ops.host(s), s_w)
 
 
-# rows kept in registers up to 8192 elements, longer ones read twice; bf16 rows in
-# one, two or four chunks a thread up to 2048, 4096, 8192
-@pytest.mark.parametrize("dim", [8192, 8196, 8200, 4, 8, 2048, 2056, 4096, 4104])
+# rows kept in registers, a chunk of 16 bytes or two, four, eight a thread: up to
+# 1024, 2048, 4096, 8192 in fp32, twice that in bf16; longer ones read twice
+@pytest.mark.parametrize("dim", [8192, 8196, 8200, 4, 8, 1024, 1028, 2048, 2052, 2056, 4096, 4104, 16384, 16392])
 def test_per_row_register_limit(oracle, ops, dim):
     x = D.normal((3, dim), 1.0, dim)
     x[1, dim - 1] = 30.0

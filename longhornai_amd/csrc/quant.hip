@@ -52,6 +52,13 @@ template <> __device__ __forceinline__ float load_f<uint16_t>(const uint16_t* p,
     return bf16_to_f32(p[i]);
 }
 
+// log2 of the threads that a workgroup gives the four-column words of a row.
+inline int column_bits(int64_t quads) {
+    int cb = 0;
+    while (cb < 8 && (int64_t{1} << cb) < quads) ++cb;
+    return cb;
+}
+
 // Quantize one value with a reciprocal (per-row / per-tensor) -- int8 or fp8.
 template <bool FP8>
 __device__ __forceinline__ uint8_t quant_mul(float x, float inv) {
@@ -214,28 +221,32 @@ __global__ __launch_bounds__(kBlock) void quant_per_row_bf16_vec_kernel(const ui
 //       a quarter of the chunk's rows, four adjacent columns per lane with
 //       16-byte loads, the waves meet in LDS, and the chunk's maxima go to
 //       dst, chunk i's at bytes [4 i cols, 4 (i + 1) cols) -- chunks are at
-//       least 64 rows, so they fit, and (3) overwrites them -- or, where one
+//       least 64 rows (or all of them), so they fit, and (3) overwrites them -- or, where one
 //       chunk holds all rows (dst may then be smaller), to the scales array.
 //       Maxima are order-independent and NaN never wins, so any split gives
 //       the reference's;
 //   (2) the maximum over the chunks, as the scale m / QMAX (1 where m == 0);
 //   (3) quantize: a thread takes its four columns' scales (and reciprocals)
-//       once and walks kQuantRows rows.
+//       once and walks R rows (8, or 2 up to 2^18 words of the matrix); a
+//       workgroup spans 4 << cb columns, all 1024 or the least power of two
+//       that holds a narrower matrix's, its other threads on further rows.
 // Bound by memory: the fp32 matrix is read twice (the second time partly
 // from the Infinity Cache) and the codes written.  K=4096, N=14336: 36 us
 // for (1) and 46 for (3); N=4097: 15 and 22.  (A thread per four columns of
 // a 64-row chunk with atomic maxima, and an IEEE division and a scale load
 // per element, took 111 us and 55 us in all.)
-// Any column count and 4-byte alignment; the last columns of a row whose
-// length is no multiple of four are taken one by one.
-constexpr int kQuantRows = 8;
-
+// Any column count and 4-byte alignment; where a row's length is no multiple
+// of four its last four columns are read and written as one word, some of them
+// twice (column by column 16 rows of 255 took twice as long).  Rows of fewer
+// than four columns are taken one by one.
 __global__ __launch_bounds__(kBlock) void col_max_kernel(const float* __restrict__ src, uint8_t* __restrict__ maxw,
                                                          int rows, int cols, int chunk) {
     __shared__ float part[4][256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c0 = blockIdx.x * 256 + lane * 4;
     const int cnt = min(4, cols - c0);  // <= 0 past the last column
+    const int w0 = cols >= 4 ? min(c0, cols - 4) : c0;  // the four columns read
+    const int last = min(cnt, 4) - 1;                   // (of fewer than four, the last one again)
     const int64_t chunks = (static_cast<int64_t>(rows) + chunk - 1) / chunk;
     // (the grid's y extent is capped, so very tall inputs give a workgroup several chunks)
     for (int64_t q = blockIdx.y; q < chunks; q += gridDim.y) {
@@ -247,17 +258,27 @@ __global__ __launch_bounds__(kBlock) void col_max_kernel(const float* __restrict
             for (int64_t r = r0; r < r1; r += 8) {
                 f32x4_t v[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = load_f32x4<full.value>(src + min(r + i, r1 - 1) * cols + c0, cnt);
+                for (int i = 0; i < 8; ++i) {
+                    const float* p = src + min(r + i, r1 - 1) * cols + w0;
+                    if constexpr (full.value) v[i] = load_f32x4<true>(p, 4);
+                    else v[i] = f32x4_t{p[0], p[min(1, last)], p[last], 0.f};
+                }
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) m[j] = amax(m[j], fabsf(v[i][j]));
             }
         };
-        if (cnt >= 4) scan(Full{});
+        if (cols >= 4) scan(Full{});
         else if (cnt > 0) scan(Part{});
         __syncthreads();
-        *reinterpret_cast<f32x4_t*>(&part[wave][lane * 4]) = f32x4_t{m[0], m[1], m[2], m[3]};
+        if (w0 == c0) {
+            *reinterpret_cast<f32x4_t*>(&part[wave][lane * 4]) = f32x4_t{m[0], m[1], m[2], m[3]};
+        } else {
+#pragma unroll
+            for (int j = 1; j < 4; ++j)
+                if (j >= c0 - w0) part[wave][lane * 4 + j - (c0 - w0)] = m[j];
+        }
         __syncthreads();
         const int c = blockIdx.x * 256 + static_cast<int>(threadIdx.x);
         float t = part[0][threadIdx.x];
@@ -295,27 +316,33 @@ __global__ __launch_bounds__(kBlock) void col_scale_kernel(const uint8_t* maxw, 
 }
 
 // q = round(x / scale[c]).
-template <bool FP8>
+template <bool FP8, int R>
 __global__ __launch_bounds__(kBlock) void quant_per_col_kernel(const float* __restrict__ src,
                                                                const float* __restrict__ scales,
-                                                               uint8_t* __restrict__ dst, int rows, int cols) {
-    const int c0 = (blockIdx.x * kBlock + threadIdx.x) * 4;
+                                                               uint8_t* __restrict__ dst, int rows, int cols,
+                                                               int cb) {
+    const int c0 = static_cast<int>(((blockIdx.x << cb) + (threadIdx.x & ((1u << cb) - 1))) * 4);
     if (c0 >= cols) return;
+    const int sub = kBlock >> cb;  // row groups of a workgroup
     const int cnt = min(4, cols - c0);
+    const int w0 = cols >= 4 ? min(c0, cols - 4) : c0;  // a ragged row's last word overlaps the one before
     auto body = [&](auto full) {
-        const f32x4_t sc = load_f32x4<full.value>(scales + c0, cnt);
+        const f32x4_t sc = load_f32x4<full.value>(scales + w0, cnt);
         f32x4_t rs;
 #pragma unroll
         for (int j = 0; j < 4; ++j) rs[j] = __builtin_amdgcn_rcpf(sc[j]);
-        for (int64_t r0 = static_cast<int64_t>(blockIdx.y) * kQuantRows; r0 < rows;
-             r0 += static_cast<int64_t>(gridDim.y) * kQuantRows) {
+        for (int64_t r0 = (static_cast<int64_t>(blockIdx.y) * sub + (threadIdx.x >> cb)) * R; r0 < rows;
+             r0 += static_cast<int64_t>(gridDim.y) * sub * R) {
             const int64_t left = rows - r0;
-            f32x4_t v[kQuantRows];
+            f32x4_t v[R];
 #pragma unroll
-            for (int i = 0; i < kQuantRows; ++i)
-                v[i] = load_f32x4<full.value>(src + (r0 + min<int64_t>(i, left - 1)) * cols + c0, cnt);
+            for (int i = 0; i < R; ++i) {
+                const float* p = src + (r0 + min<int64_t>(i, left - 1)) * cols + w0;
+                if constexpr (full.value) v[i] = load_f32x4<true>(p, 4);
+                else v[i] = f32x4_t{p[0], p[min(1, cnt - 1)], p[cnt - 1], 0.f};
+            }
 #pragma unroll
-            for (int i = 0; i < kQuantRows; ++i) {
+            for (int i = 0; i < R; ++i) {
                 if (i >= left) break;
                 uint32_t o = 0;
                 if constexpr (FP8) {
@@ -329,11 +356,11 @@ __global__ __launch_bounds__(kBlock) void quant_per_col_kernel(const float* __re
                         o |= (static_cast<uint32_t>(sat_rint(t, 127)) & 0xffu) << (8 * j);
                     }
                 }
-                store_u8x4<full.value>(dst + (r0 + i) * cols + c0, o, cnt);
+                store_u8x4<full.value>(dst + (r0 + i) * cols + w0, o, cnt);
             }
         }
     };
-    if (cnt == 4) body(Full{});
+    if (cols >= 4) body(Full{});
     else body(Part{});
 }
 
@@ -800,7 +827,10 @@ int quantize_per_col(const float* src, uint8_t* dst, float* scales, int rows, in
     hipStream_t s = as_stream(stream);
     // long chunks (little to merge) where they still make four workgroups per CU
     const int64_t strips = ceil_div(cols, 256);
-    const int chunk = strips * ceil_div(rows, 256) >= 1024 ? 256 : strips * ceil_div(rows, 128) >= 1024 ? 128 : 64;
+    const int chunk = rows < 64                                ? max(4, ceil_div(rows, 4) * 4)
+                      : strips * ceil_div(rows, 256) >= 1024 ? 256
+                      : strips * ceil_div(rows, 128) >= 1024 ? 128
+                                                             : 64;
     const int chunks = ceil_div(rows, chunk);
     uint8_t* const maxw = chunks > 1 ? dst : reinterpret_cast<uint8_t*>(scales);
     if (rows > 0)
@@ -808,9 +838,13 @@ int quantize_per_col(const float* src, uint8_t* dst, float* scales, int rows, in
             src, maxw, rows, cols, chunk);
     col_scale_kernel<FP8><<<blocks_for(cols, 64), kBlock, 0, s>>>(maxw, chunks, scales, cols);
     if (rows > 0) {
-        const dim3 grid(static_cast<unsigned>(ceil_div(ceil_div(cols, 4), kBlock)),
-                        static_cast<unsigned>(min(ceil_div(rows, kQuantRows), 65535)));
-        quant_per_col_kernel<FP8><<<grid, kBlock, 0, s>>>(src, scales, dst, rows, cols);
+        const int64_t quads = ceil_div64(cols, 4);
+        const int cb = column_bits(quads);
+        const int r = quads * rows > (1 << 18) ? 8 : 2;
+        const dim3 grid(static_cast<unsigned>(ceil_div64(quads, int64_t{1} << cb)),
+                        static_cast<unsigned>(min(ceil_div(rows, r * (kBlock >> cb)), 65535)));
+        if (r == 8) quant_per_col_kernel<FP8, 8><<<grid, kBlock, 0, s>>>(src, scales, dst, rows, cols, cb);
+        else quant_per_col_kernel<FP8, 2><<<grid, kBlock, 0, s>>>(src, scales, dst, rows, cols, cb);
     }
     return check_launch(who);
 }

@@ -99,8 +99,10 @@ def test_per_tensor_empty(ops):
     assert ops.host(s)[0] == 1.0
 
 
-# one row chunk (any height below 64 rows), a chunk's edges, two column blocks
-@pytest.mark.parametrize("rows,cols", [(1, 5), (2, 1030), (63, 258), (64, 3), (129, 257), (1000, 7)])
+# one row chunk (any height below 64 rows), a chunk's edges, two column blocks, a
+# last word across a block's edge, narrow matrices, two and eight rows a thread
+@pytest.mark.parametrize("rows,cols", [(1, 5), (2, 1030), (63, 258), (64, 3), (129, 257), (1000, 7), (16, 255), (5, 1), (9, 2),
+                                       (70, 259), (2100, 510), (1025, 1030), (1 << 18, 3), ((1 << 18) + 9, 3)])
 @pytest.mark.parametrize("kind", ["q8", "fp8"])
 def test_per_col(oracle, ops, rows, cols, kind):
     x = _weights(rows, cols, rows * cols) if rows > 1 else D.normal((rows, cols), 1.0, cols)

@@ -583,20 +583,28 @@ __global__ void q4a_pack_kernel(const float* __restrict__ src, const uint16_t* _
     packed[t] = static_cast<uint8_t>(b);
 }
 
-// Dequantize int4: a thread owns four adjacent columns and kDeqPairs packed
-// rows, reading a 32-bit word of codes and writing two 16-byte runs of fp32
-// per packed row.  Bound by the write: K=4096, N=14336, G=128 writes 235 MB
-// in 44 us (a thread per element with two 64-bit divisions took 117).
-constexpr int kDeqPairs = 4;
-
-template <bool ASYM>
+// Dequantize int4: a thread owns four adjacent columns and P packed rows,
+// reading a 32-bit word of codes and writing two 16-byte runs of fp32 per
+// packed row.  Bound by the write: K=4096, N=14336, G=128 writes 235 MB in 44
+// us (a thread per element with two 64-bit divisions took 117).
+// P is 4, and 1 up to 2^18 words of codes, where four rows a thread took 1.1
+// to 1.5 times as long in the mean (K=64, N=8192 3.15 us, one row 2.19; K=2048,
+// N=8192 one row 13.5, four 14.1 or as little as 0.82 of one).
+// A workgroup spans 4 << cb columns: all 1024, or for narrower weights the
+// least power of two that holds them, its other threads on further rows.
+// Where N is no multiple of four a row's last four columns are one word too,
+// some of them written twice (K=1024, N=411 2.2 us; 5.6 one by one); fewer than
+// four columns are taken one by one.
+template <bool ASYM, int P>
 __global__ __launch_bounds__(kBlock) void q4_dequant_kernel(const uint8_t* __restrict__ packed,
                                                             const void* __restrict__ scales,
                                                             const uint8_t* __restrict__ zeros,
-                                                            float* __restrict__ dst, int K, int N, int G) {
-    const int c0 = (blockIdx.x * kBlock + threadIdx.x) * 4;
-    if (c0 >= N) return;
-    const int cnt = min(4, N - c0);
+                                                            float* __restrict__ dst, int K, int N, int G, int cb) {
+    const int c = static_cast<int>(((blockIdx.x << cb) + (threadIdx.x & ((1u << cb) - 1))) * 4);
+    if (c >= N) return;
+    const int cnt = min(4, N - c);
+    const int c0 = N >= 4 ? min(c, N - 4) : c;
+    const int sub = kBlock >> cb;  // row groups of a workgroup
     struct Params {
         f32x4_t s;
         uint32_t z;
@@ -608,9 +616,16 @@ __global__ __launch_bounds__(kBlock) void q4_dequant_kernel(const uint8_t* __res
             Params p = {{0.f, 0.f, 0.f, 0.f}, 0u};
             if constexpr (ASYM) {
                 const uint16_t* sp = static_cast<const uint16_t*>(scales) + gi;
+                if constexpr (F) {
+                    uint16_t h[4];
+                    __builtin_memcpy(h, sp, 8);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (F || j < cnt) p.s[j] = f16_to_f32(sp[j]);
+                    for (int j = 0; j < 4; ++j) p.s[j] = f16_to_f32(h[j]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (j < cnt) p.s[j] = f16_to_f32(sp[j]);
+                }
                 p.z = load_u8x4<F>(zeros + gi, cnt);
             } else {
                 p.s = load_f32x4<F>(static_cast<const float*>(scales) + gi, cnt);
@@ -629,18 +644,18 @@ __global__ __launch_bounds__(kBlock) void q4_dequant_kernel(const uint8_t* __res
             store_f32x4<F>(dst + k * N + c0, v, cnt);
         };
         const int pairs = K / 2;
-        for (int64_t i0 = static_cast<int64_t>(blockIdx.y) * kDeqPairs; i0 < pairs;
-             i0 += static_cast<int64_t>(gridDim.y) * kDeqPairs) {
-            uint32_t w[kDeqPairs];
-            Params p[kDeqPairs];
+        for (int64_t i0 = (static_cast<int64_t>(blockIdx.y) * sub + (threadIdx.x >> cb)) * P; i0 < pairs;
+             i0 += static_cast<int64_t>(gridDim.y) * sub * P) {
+            uint32_t w[P];
+            Params p[P];
 #pragma unroll
-            for (int u = 0; u < kDeqPairs; ++u) {
+            for (int u = 0; u < P; ++u) {
                 const int64_t i = i0 + u < pairs ? i0 + u : pairs - 1;
                 w[u] = load_u8x4<F>(packed + i * N + c0, cnt);
                 p[u] = params(static_cast<int>(2 * i) / G);
             }
 #pragma unroll
-            for (int u = 0; u < kDeqPairs; ++u) {
+            for (int u = 0; u < P; ++u) {
                 if (i0 + u >= pairs) break;
                 const int k = static_cast<int>(2 * (i0 + u));
                 put(k, w[u], p[u]);
@@ -649,16 +664,20 @@ __global__ __launch_bounds__(kBlock) void q4_dequant_kernel(const uint8_t* __res
             }
         }
     };
-    if (cnt == 4) body(Full{});
+    if (N >= 4) body(Full{});
     else body(Part{});
 }
 
 template <bool ASYM>
 void launch_q4_dequant(const uint8_t* packed, const void* scales, const uint8_t* zeros, float* dst, int K, int N,
                        int G, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(ceil_div(ceil_div(N, 4), kBlock)),
-                    static_cast<unsigned>(min(ceil_div(K / 2, kDeqPairs), 65535)));
-    q4_dequant_kernel<ASYM><<<grid, kBlock, 0, s>>>(packed, scales, zeros, dst, K, N, G);
+    const int64_t quads = ceil_div64(N, 4);
+    const int cb = column_bits(quads);
+    const int p = quads * (K / 2) > (1 << 18) ? 4 : 1;
+    const dim3 grid(static_cast<unsigned>(ceil_div64(quads, int64_t{1} << cb)),
+                    static_cast<unsigned>(min(ceil_div(K / 2, p * (kBlock >> cb)), 65535)));
+    if (p == 4) q4_dequant_kernel<ASYM, 4><<<grid, kBlock, 0, s>>>(packed, scales, zeros, dst, K, N, G, cb);
+    else q4_dequant_kernel<ASYM, 1><<<grid, kBlock, 0, s>>>(packed, scales, zeros, dst, K, N, G, cb);
 }
 
 // Groups of 32, 64, 128 or 256 rows, scales and codes in one pass over the

@@ -62,7 +62,8 @@ def test_int4_groups(oracle, ops, K, N, G, lead):
     _same(ops.host(z), z_w)
 
 
-@pytest.mark.parametrize("K,N,G", [(30, 7, 3), (30, 9, 1), (64, 1027, 16), (34, 4, 2), (10, 6, 10)])
+@pytest.mark.parametrize("K,N,G", [(30, 7, 3), (30, 9, 1), (64, 1027, 16), (34, 4, 2), (10, 6, 10), (66, 1, 2), (62, 2, 1),
+                                   (516, 3, 6), (2048, 1027, 16), (2052, 1026, 9)])
 @pytest.mark.parametrize("lead", [0, 3])
 def test_int4_dequantize(oracle, ops, K, N, G, lead):
     g = D.rng(K * N + G)

@@ -173,7 +173,7 @@ def test_w4_prepack_layout(ops, K, N, G, lead):
     assert ops.host(q).tobytes() == _w4_layout(u ^ 8, K, N)
 
 
-@pytest.mark.parametrize("K,N", [(128, 128), (130, 257), (1, 3), (300, 1001)])
+@pytest.mark.parametrize("K,N", [(128, 128), (130, 257), (1, 3), (300, 1001), (128, 5), (4, 126), (700, 2), (131, 4)])
 def test_b8_prepack_layout(ops, K, N):
     b = D.rng(K + N).integers(0, 256, (K, N)).astype(np.uint8)
     bt = ops.prepack_b8(_off(ops, b, 1), K, N)

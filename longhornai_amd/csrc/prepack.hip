@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void w4_prepack_kernel(const uint8_t* __restri
                                                          const uint8_t* __restrict__ zeros,
                                                          uint32_t* __restrict__ zeros_out, int K, int N, int Nt,
                                                          int Kt, int NG, int64_t qblocks, int64_t sblocks) {
-    const int64_t blk = blockIdx.x;
+    const int64_t blk = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
     if (blk < qblocks) {
         const int kt = static_cast<int>(blk % Kt);
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void w4_prepack_kernel(const uint8_t* __restri
                 w4_quad(r, d[j]);
             }
         };
-        if (n0 + 4 <= N) read(Full{});
+        if (n0 <= N - 4) read(Full{});
         else read(Part{});
         u32x4_t* o = reinterpret_cast<u32x4_t*>(qweight + (static_cast<int64_t>(nt) * Kt + kt) * kW4TileBytes) +
                      16 * kq + 4 * (c4 & 3);
@@ -120,7 +120,10 @@ int launch_w4_prepack(const uint8_t* packed, const S* scales, const uint8_t* zer
     const int64_t qb = static_cast<int64_t>(ceil_div(Nt, 16)) * Kt;
     const int64_t sb = ceil_div64(static_cast<int64_t>(Nt) * NG * 16, 256);
     const int64_t zb = ASYM ? ceil_div64(static_cast<int64_t>(Nt) * ceil_div(NG, 8) * 16, 256) : 0;
-    w4_prepack_kernel<ASYM, S><<<static_cast<unsigned>(qb + sb + zb), 256, 0, s>>>(
+    // a second grid dimension past 2^30 threads; the blocks past the last one end
+    // in the last section's own bounds
+    const int64_t total = qb + sb + zb, gx = total < (1 << 22) ? total : 1 << 22;
+    w4_prepack_kernel<ASYM, S><<<dim3(static_cast<unsigned>(gx), static_cast<unsigned>(ceil_div64(total, gx))), 256, 0, s>>>(
         packed, qweight, scales, scales_out, zeros, zeros_out, K, N, Nt, Kt, NG, qb, sb);
     return check_launch(who);
 }

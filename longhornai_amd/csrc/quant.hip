@@ -760,7 +760,7 @@ template <bool ASYM>
 bool launch_q4_group(const float* src, void* scales, uint8_t* zeros, uint8_t* packed, int K, int N, int G,
                      hipStream_t s) {
     const int NG = K / G;
-    const dim3 grid(static_cast<unsigned>(ceil_div(N, 64)), static_cast<unsigned>(min(NG, 65535)));
+    const dim3 grid(static_cast<unsigned>(ceil_div64(N, 64)), static_cast<unsigned>(min(NG, 65535)));
     if (G == 32) q4_group_kernel<ASYM, 8><<<grid, 256, 0, s>>>(src, scales, zeros, packed, N, NG);
     else if (G == 64) q4_group_kernel<ASYM, 16><<<grid, 256, 0, s>>>(src, scales, zeros, packed, N, NG);
     else if (G == 128) q4_group_kernel<ASYM, 32><<<grid, 256, 0, s>>>(src, scales, zeros, packed, N, NG);
@@ -845,12 +845,12 @@ int quantize_per_col(const float* src, uint8_t* dst, float* scales, int rows, in
     if (cols == 0) return LHQ_OK;
     hipStream_t s = as_stream(stream);
     // long chunks (little to merge) where they still make four workgroups per CU
-    const int64_t strips = ceil_div(cols, 256);
+    const int64_t strips = ceil_div64(cols, 256);
     const int chunk = rows < 64                                ? max(4, ceil_div(rows, 4) * 4)
-                      : strips * ceil_div(rows, 256) >= 1024 ? 256
-                      : strips * ceil_div(rows, 128) >= 1024 ? 128
+                      : strips * ceil_div64(rows, 256) >= 1024 ? 256
+                      : strips * ceil_div64(rows, 128) >= 1024 ? 128
                                                              : 64;
-    const int chunks = ceil_div(rows, chunk);
+    const int chunks = static_cast<int>(ceil_div64(rows, chunk));
     uint8_t* const maxw = chunks > 1 ? dst : reinterpret_cast<uint8_t*>(scales);
     if (rows > 0)
         col_max_kernel<<<dim3(static_cast<unsigned>(strips), static_cast<unsigned>(min(chunks, 65535))), kBlock, 0, s>>>(
@@ -861,7 +861,7 @@ int quantize_per_col(const float* src, uint8_t* dst, float* scales, int rows, in
         const int cb = column_bits(quads);
         const int r = quads * rows > (1 << 18) ? 8 : 2;
         const dim3 grid(static_cast<unsigned>(ceil_div64(quads, int64_t{1} << cb)),
-                        static_cast<unsigned>(min(ceil_div(rows, r * (kBlock >> cb)), 65535)));
+                        static_cast<unsigned>(std::min<int64_t>(ceil_div64(rows, r * (kBlock >> cb)), 65535)));
         if (r == 8) quant_per_col_kernel<FP8, 8><<<grid, kBlock, 0, s>>>(src, scales, dst, rows, cols, cb);
         else quant_per_col_kernel<FP8, 2><<<grid, kBlock, 0, s>>>(src, scales, dst, rows, cols, cb);
     }

@@ -137,6 +137,23 @@ def test_per_row_register_limit(oracle, ops, dim):
     _same(ops.host(s), s_w)
 
 
+def test_sizes_near_two_to_the_31(ops):
+    n = (1 << 31) - 1
+    x = ops.zeros((n,), np.float32)
+    x[n - 1], x[5] = 50.0, -25.0
+    q, s = ops.empty((n,), np.int8), ops.empty((1,), np.float32)
+    ops.run("lhq_q8_quantize_per_col", x, q, s, n, 1)
+    assert ops.host(s)[0] == np.float32(50.0) / np.float32(127.0)
+    assert int((q != 0).sum()) == 2 and int(q[n - 1]) == 127 and int(q[5]) == -64
+    x.fill_(0.5)
+    x[n - 1] = 3.0
+    p, d = ops.zeros((n,), np.uint8), ops.empty((2 * n,), np.float32)
+    p[n - 1], p[0] = 0x7A, 0x01
+    ops.run("lhq_q4_dequantize_groupwise", p, x, d, 2, n, 2)
+    assert int((d != 0).sum()) == 3
+    assert float(d[n - 1]) == -18.0 and float(d[2 * n - 1]) == 21.0 and float(d[0]) == 0.5
+
+
 def _w4_layout(codes, K, N):
     """[Nt][Kt][64][16 B]: lane l, dword j, element e at nibble w4_slot(e)."""
     Nt, Kt = -(-N // 16), -(-K // 128)

@@ -386,6 +386,9 @@ int lhq_gemm_f32_batched(const float* A, const float* B, float* C, int batch, in
  * reference's rule (dtypes.hpp:87-98).  counts: 2 device uint64, set to
  * {non-NaN mismatches, NaN mismatches}; both are 0 on a conforming device. */
 int lhq_selftest_bf16(unsigned long long* counts, void* stream);
+/* The same for E4M3: the pair conversion the quantizers use against the
+ * reference's rule (dtypes.hpp:111-158) one value at a time; counts pairs. */
+int lhq_selftest_e4m3(unsigned long long* counts, void* stream);
 /* The form of the W4A16 kernel for a few rows (weights streamed, rows staged
  * on chip) that this call takes on the current device with 16-byte aligned
  * activations: 16 * (16-row blocks) + column tiles per workgroup, 0 where

@@ -88,6 +88,7 @@ SIGNATURES = {
     "lhq_gemm_f32_ref": [_p, _p, _p, _i, _i, _i, _f, _f, _p],
     "lhq_gemm_f32_batched": [_p, _p, _p, _i, _i, _i, _i, _f, _f, _p],
     "lhq_selftest_bf16": [_p, _p],
+    "lhq_selftest_e4m3": [_p, _p],
     "lhq_selftest_w4_stream": [_i, _i, _i, _i, _i],
     "lhq_selftest_gemm8_stream": [_i, _i, _i, _i],
 }

@@ -181,7 +181,7 @@ __device__ __forceinline__ uint8_t f32_to_e4m3(float value) {
 // 8..15 of the result): the conversion rounds to nearest even with
 // denormals; saturation, the flush below 2^-9, NaN / inf and the sign are
 // made around it.  Equal to f32_to_e4m3 for every one of the 2^32 inputs
-// (checked on the device); about a third of its instructions.
+// (lhq_selftest_e4m3 runs them); about a third of its instructions.
 __device__ __forceinline__ uint32_t pack_e4m3x2(float a, float b) {
     const float ma = fabsf(a), mb = fabsf(b);
     const uint32_t w = static_cast<uint32_t>(

@@ -2080,12 +2080,10 @@ __global__ __launch_bounds__(L >= 3 ? 512 : 256, L == 3 ? 1 : 2) void w4_mma_ker
 // the partial sums of workers wa..wb in slots wa + tr .. wb + tr, added in
 // that (K) order and written as the tile kernel writes a tile.  Workgroup
 // 4 tr + qn takes column quarter qn of the tile (the 16 KiB a slot holds for
-// wave qn): thread t holds lane t & 63 of column tile t >> 6 at row blocks
-// 0..3, or with SWI the gate / up pair (2 (t >> 6 & 1), + 1) at row blocks
-// 2 (t >> 7) and + 1; each segment's loads are issued four segments at a
-// time before they are added.  W32 (slots written by mma_tile32): thread t
-// holds lane t & 63 of blocks (ib, cb) at the D rows 8 i4 .. of the (ib, i4)
-// pairs 2 (t >> 6) and + 1, cb = 0 and 1 of each (a gate / up pair with SWI).
+// wave qn, as mma_tile32 wrote them): thread t holds lane t & 63 of blocks
+// (ib, cb) at the D rows 8 i4 .. of the (ib, i4) pairs 2 (t >> 6) and + 1,
+// cb = 0 and 1 of each (a gate / up pair with SWI); each segment's loads are
+// issued four segments at a time before they are added.
 template <bool SWI>
 __global__ __launch_bounds__(256) void w4_pk_fixup_kernel(W4Args p) {
     const PkPlan pl = pk_plan(p, p.pk_workers);

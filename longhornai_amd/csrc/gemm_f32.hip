@@ -208,8 +208,8 @@ void launch_tile(const float* A, const float* B, float* C, int batch, int M, int
 // M=128, N=1024 6.8 / 3.1; K=80, M=2000, N=2048 19.9 / 22.8; M=2000, N=8192: K=96
 // 64 / 75, K=192 111 / 115, K=256 142 / 130.  By valu_wins both together are
 // 2.87 and 3.08 times as fast as this one alone over a grid of 2,184 shapes and
-// 2,500 random ones, one of them more than 2.5% slower (131 x 38 x 192 x 16
-// (M, K, N, batch) 8.9 / 9.4).
+// 2,500 random ones, three of them more than 2.5% slower, by 5% at most (131 x 38
+// x 192 x 16 (M, K, N, batch) 8.9 / 9.4).
 // Its grid has two dimensions for the outputs, so it also takes those past
 // 2^32 threads of the other's one.
 constexpr int T = 64, TK = 16;
